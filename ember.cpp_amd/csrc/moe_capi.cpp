@@ -23,11 +23,14 @@ namespace {
 constexpr int kMaxE = 512;  // route_kernel keeps one bit per (lane, 64-expert stripe) and LDS rows of E
 constexpr int kMaxK = 64;   // picks live in a 64-entry LDS array per wave
 // Expert-product kernels by tokens per expert (M): the int16-dot GEMV while M is at most a few tokens,
-// the skinny MFMA GEMM (64-token tiles) for up to ~100, the 256-token-tile MFMA GEMM beyond.
+// the skinny MFMA GEMM (64-token tiles) for up to ~100, the 256-token-tile MFMA GEMM beyond. F32 stacks: the
+// GEMV, then the FP32 MFMA tiles (64 tokens) at any size.
 enum PathMode { kGemv = 0, kSkinny = 1, kGemm = 2 };
+bool f32_stacks(int type_in, int type_out) { return type_in == EMBER_TYPE_F32 && type_out == EMBER_TYPE_F32; }
 int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int E, bool packed = false,
               bool with_shared = false) {
-  if (!gemm_supported(type_in, K_in) || !gemm_supported(type_out, K_out)) return kGemv;
+  const bool f32 = f32_stacks(type_in, type_out);  // tiles on the FP32 matrix cores (moe_gemm_f32.hip)
+  if (!f32 && (!gemm_supported(type_in, K_in) || !gemm_supported(type_out, K_out))) return kGemv;
   // tuning override: gemv | skinny | gemm (read per call, so a test can select each kernel); the shared
   // expert (E = 1 here) reads EMBER_MOE_SHARED_PATH
   const int forced = [E] {
@@ -36,6 +39,7 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
     const std::string s(v);
     return s == "gemv" ? kGemv : s == "skinny" ? kSkinny : s == "gemm" ? kGemm : -1;
   }();
+  if (f32 && forced >= 0) return forced == kGemv ? kGemv : kSkinny;
   if (forced >= 0) return forced;
   // Q8_0 (its DMA tile kernels): the GEMV up to 1 token per expert with the prefill pack, 2 without,
   // then the 256-token-tile kernel, which skips the empty 32-row subtiles of a short segment (C2 with the
@@ -51,6 +55,18 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
   const double slots = avg_m * E;
   const double hit = slots > 0.0 ? E * (1.0 - std::pow(1.0 - 1.0 / E, slots)) : 0.0;
   const double per_hit = hit > 0.0 ? slots / hit : 0.0;
+  // F32: the GEMV up to 2.6 tokens per hit expert (GEMV / tiles, d 1024, d_ff 2816, E 8: T = 8 (2.3) 92 / 99
+  // us, T = 10 (2.6) 105 / 105, T = 12 112 / 105, T = 64 322 / 112, T = 400 1721 / 221), up to 1.8 when the
+  // layer's stacks exceed 1 GB and a second pass over them costs the most (Mixtral-shaped T = 4 (1.5) 817 / 1060,
+  // T = 6 (1.9) 1201 / 1177, T = 8 1441 / 1204, T = 128 17179 / 1770; Qwen-shaped T = 16 (1.5) 399 / 411, T =
+  // 24 (1.9) 547 / 487), up to 3.5 when they are under 32 MB and launches and latency set the time (d 256, d_ff
+  // 688, E 8: T = 12 (3.1) 42 / 45, T = 16 (4) 46 / 45, T = 512 497 / 71). A dense shared expert, whose few
+  // tiles leave most CUs idle in a small batch, up to 64 rows.
+  if (f32) {
+    const int64_t bytes = (int64_t)E * 12 * K_in * K_out;
+    const double most = bytes < ((int64_t)32 << 20) ? 3.5 : bytes > ((int64_t)1 << 30) ? 1.8 : 2.6;
+    return (E == 1 ? avg_m <= 64.0 : per_hit <= most) ? kGemv : kSkinny;
+  }
   // packed Q4_K (the same DMA tile kernels): the GEMV up to 1.55 tokens per hit expert, then the
   // 256-token tiles (Qwen-shaped E = 128, GEMV / 64-token / 256-token tiles: T = 13 (1.47) 114 / 119 / 116
   // us, T = 14 (1.51) 122 / 119 / 114, T = 16 (1.58) 128 / 118 / 115, T = 24 170 / 155 / 150, T = 48 255 /
@@ -246,7 +262,10 @@ Layout layout(const ember_moe_layer* w, int T) {
   // the shared expert's dense launches on 64-token tiles have d_ff_shared / 128 (gate/up) and d / 256
   // (down) blocks per 64 tokens: split over K until the chip is filled (C4 shape, T = 16: 128 -> 25 us)
   l.ks_sh_gu = l.ks_sh_dn = 1;
-  if (w->d_ff_shared > 0 && l.mode_shared == kSkinny) {
+  const bool f32_sh = w->d_ff_shared > 0 && f32_stacks(w->gate_shared_type, w->down_shared_type);
+  if (w->d_ff_shared > 0 && l.mode_shared == kSkinny && f32_sh) {
+    l.ks_sh_dn = gemm_f32_ksplit((T + 63) / 64, w->d, w->d_ff_shared);
+  } else if (w->d_ff_shared > 0 && l.mode_shared == kSkinny) {
     l.ks_sh_gu = gemm_dense_ksplit(true, T, w->d_ff_shared, w->d,
                                    2 * (int64_t)w->d_ff_shared * row_bytes(w->gate_shared_type, w->d));
     l.ks_sh_dn = gemm_dense_ksplit(false, T, w->d, w->d_ff_shared,
@@ -257,7 +276,9 @@ Layout layout(const ember_moe_layer* w, int T) {
   const size_t tiles = l.mode == kGemm     ? (size_t)gemm_max_tiles(T, w->k, w->E)
                        : l.mode == kSkinny ? (size_t)gemm_skinny_max_tiles(T, w->k, w->E)
                                            : 0;
-  const bool mfma = l.mode != kGemv, mfma_sh = w->d_ff_shared > 0 && l.mode_shared != kGemv;
+  // (the F32 tiles read x and write h in f32: none of the converted activations below)
+  const bool mfma = l.mode != kGemv && !f32_stacks(w->gate_type, w->down_type);
+  const bool mfma_sh = w->d_ff_shared > 0 && l.mode_shared != kGemv && !f32_sh;
   const bool sp = split_bf16(w->gate_type, w->down_type) && !pack_bf16;
   const bool sp_sh = w->d_ff_shared > 0 && split_bf16(w->gate_shared_type, w->down_shared_type) &&
                      !(pack_bf16 && bf16_shared(w));
@@ -485,9 +506,12 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
   conv.x = x;
   conv.rows = T;
   conv.K = d;
-  conv.y16 = (l.mode != kGemv && !sp) || (shared_mfma && !sp_sh) ? x16 : nullptr;
+  const bool f32 = f32_stacks(w->gate_type, w->down_type);
+  const bool f32_sh = shared && f32_stacks(w->gate_shared_type, w->down_shared_type);
+  const bool half_act = l.mode != kGemv && !f32, half_act_sh = shared_mfma && !f32_sh;
+  conv.y16 = (half_act && !sp) || (half_act_sh && !sp_sh) ? x16 : nullptr;
   conv.yexp = xexp;
-  conv.yb = (l.mode != kGemv && sp) || (shared_mfma && sp_sh) ? xb : nullptr;
+  conv.yb = (half_act && sp) || (half_act_sh && sp_sh) ? xb : nullptr;
   conv.plane = (int64_t)T * d;
   const bool need_conv = conv.y16 || conv.yb;
   auto* flag = at<unsigned long long>(scratch, l.flag);
@@ -525,6 +549,28 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
   // idle (their tail rounds) instead of running alone on a few hundred blocks.
   auto run_shared = [&](hipStream_t sst) -> int {
     int s = EMBER_OK;
+    if (f32_sh) {
+      GemmF32Args g{};
+      g.A = x;
+      g.T = T;
+      g.W0 = static_cast<const float*>(w->gate_shared);
+      g.W1 = static_cast<const float*>(w->up_shared);
+      g.N = w->d_ff_shared;
+      g.K = d;
+      g.out = hs;
+      g.ksplit = 1;
+      const int mt = gemm_skinny_max_tiles(T, 1, 0);
+      if ((s = launch_gemm_f32(g, true, mt, sst))) return s;
+      g.A = hs;
+      g.W0 = static_cast<const float*>(w->down_shared);
+      g.W1 = nullptr;
+      g.N = d;
+      g.K = w->d_ff_shared;
+      g.out = ys;
+      g.ksplit = l.ks_sh_dn;
+      g.part_stride = (int64_t)T * d;
+      return launch_gemm_f32(g, false, mt, sst);
+    }
     _Float16* hs16 = at<_Float16>(scratch, l.hs16);
     int32_t* hsexp = at<int32_t>(scratch, l.hsexp);
     GemmArgs g{};
@@ -595,7 +641,36 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     if ((s = run_shared(side->s))) return s;
   }
 
-  if (l.mode != kGemv) {
+  if (l.mode != kGemv && f32) {
+    GemmF32Args g{};
+    g.A = x;
+    g.perm = perm;
+    g.k = k;
+    g.T = T;
+    g.W0 = static_cast<const float*>(w->gate);
+    g.W1 = static_cast<const float*>(w->up);
+    g.N = d_ff;
+    g.K = d;
+    g.tiles = ds.tiles;
+    g.n_tiles = ds.n_tiles;
+    g.offsets = offsets;
+    g.out = h;
+    g.ksplit = 1;
+    const int mt = gemm_skinny_max_tiles(T, k, E);
+    if ((s = launch_gemm_f32(g, true, mt, st))) return s;
+    mark(ev, 4, st);
+    g.A = h;
+    g.perm = nullptr;
+    g.W0 = static_cast<const float*>(w->down);
+    g.W1 = nullptr;
+    g.N = d;
+    g.K = d_ff;
+    g.out = y;
+    g.ksplit = ksplit = gemm_f32_ksplit(gemm_expected_tiles(T, k, E), d, d_ff);
+    g.part_stride = (int64_t)T * k * d;
+    if ((s = launch_gemm_f32(g, false, mt, st))) return s;
+    mark(ev, 5, st);
+  } else if (l.mode != kGemv) {
     const bool skinny = l.mode == kSkinny;
     auto gemm = [&](const GemmArgs& g, bool gated, int mt) {
       return skinny ? launch_gemm_skinny(g, gated, mt, st) : launch_gemm(g, gated, mt, st);

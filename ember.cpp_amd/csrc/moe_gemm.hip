@@ -10,7 +10,7 @@
 // Q4_K: (d*sc)*q - dmin*m by one fused multiply-add of the fp16-rounded factors; BF16: RNE to fp16),
 // activations are fp16, products accumulate in fp32 on v_mfma_f32_32x32x16_f16. The relative error
 // of a layer is ~4e-4 (rel-L2), inside the 2e-3 bar for quantized stacks. F32 stacks never take this
-// path (their bar is 1e-5).
+// path (their bar is 1e-5): moe_gemm_f32.hip.
 //
 // Kernels: gemm_dma_q8_kernel (Q8_0 rows or the prefill pack's Q8_0 / Q4_K tiles; 256-token tiles,
 // weights and activations loaded straight into LDS), gemm_dma64_q8_kernel (the same formats, 64-token
@@ -1468,6 +1468,8 @@ static double expected_row_tiles(int T, int k, int E, int bm) {
     per_e += sd > 0 ? 0.5 * std::erfc((bm * j + 0.5 - m) / (sd * std::sqrt(2.0))) : (m > bm * j ? 1.0 : 0.0);
   return E * per_e;
 }
+
+int gemm_expected_tiles(int T, int k, int E) { return (int)std::ceil(expected_row_tiles(T, k, E, SBM)); }
 
 int gemm_ksplit(int type, bool packed, int T, int k, int E, int N, int K) {
   if (!dma_path(type, packed)) return 1;  // the split lives in the DMA kernels

@@ -253,6 +253,25 @@ struct GemmArgs {
   // finished by gemm_tail_fixup_kernel. tail_parts <= 1: no split.
   int tail_parts, slots;
 };
+// Grouped GEMM over F32 stacks on the FP32 matrix cores (moe_gemm_f32.hip): tiles as in GemmArgs, of 64 tokens
+// (gemm_tile_rows(true)), or T dense rows when tiles is null. Any K and N that are multiples of 4.
+struct GemmF32Args {
+  const float* A;          // activation rows [*][K]
+  const int32_t* perm;     // non-null: row of sorted position p is perm[p] / k
+  int k, T;
+  const float* W0;         // gate (or the only) stack [E][N][K]
+  const float* W1;         // up stack (gated) or null
+  int N, K;
+  const int32_t* tiles;
+  const int32_t* n_tiles;
+  const int32_t* offsets;
+  float* out;              // gated: h [pos][N]; plain: y [pos][N], part s at + s * part_stride
+  int ksplit;              // plain projections: K split over this many blocks (1 when gated)
+  int64_t part_stride;
+};
+int launch_gemm_f32(const GemmF32Args& g, bool gated, int max_mtiles, hipStream_t st);
+// K split of a plain projection of about `mtiles` 64-token tiles: 1 .. kMaxKSplit
+int gemm_f32_ksplit(int mtiles, int N, int K);
 // Parts of the tail split (GemmArgs::tail_parts) for a gated 256-token-tile launch of T k rows against
 // N = d_ff columns over K = d: 0 when it does not apply (the partials' size bound); and the resident blocks
 // per round (a multiple of 8).
@@ -329,6 +348,7 @@ int gemm_tile_rows(bool skinny);
 // Skinny variant for segments of a few dozen tokens (64-token tiles).
 int launch_gemm_skinny(const GemmArgs& g, bool gated, int max_mtiles, hipStream_t st);
 int gemm_skinny_max_tiles(int T, int k, int E);
+int gemm_expected_tiles(int T, int k, int E);  // 64-token tiles of uniform routing, rounded up
 // K split of the skinny path's plain (down) projection: 1..kMaxKSplit, so that the launch has enough
 // blocks for the chip when the output is narrow
 constexpr int kMaxKSplit = 4;
