@@ -55,16 +55,16 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
   const double slots = avg_m * E;
   const double hit = slots > 0.0 ? E * (1.0 - std::pow(1.0 - 1.0 / E, slots)) : 0.0;
   const double per_hit = hit > 0.0 ? slots / hit : 0.0;
-  // F32: the GEMV up to 2.6 tokens per hit expert (GEMV / tiles, d 1024, d_ff 2816, E 8: T = 8 (2.3) 92 / 99
-  // us, T = 10 (2.6) 105 / 105, T = 12 112 / 105, T = 64 322 / 112, T = 400 1721 / 221), up to 1.8 when the
-  // layer's stacks exceed 1 GB and a second pass over them costs the most (Mixtral-shaped T = 4 (1.5) 817 / 1060,
-  // T = 6 (1.9) 1201 / 1177, T = 8 1441 / 1204, T = 128 17179 / 1770; Qwen-shaped T = 16 (1.5) 399 / 411, T =
-  // 24 (1.9) 547 / 487), up to 3.5 when they are under 32 MB and launches and latency set the time (d 256, d_ff
-  // 688, E 8: T = 12 (3.1) 42 / 45, T = 16 (4) 46 / 45, T = 512 497 / 71). A dense shared expert, whose few
-  // tiles leave most CUs idle in a small batch, up to 64 rows.
+  // F32: the GEMV up to 2.6 tokens per hit expert (GEMV / tiles, d 1024, d_ff 2816, E 8: T = 8 (2.3) 92 / 97
+  // us, T = 10 (2.7) 104 / 102, T = 64 322 / 106, T = 400 1719 / 223), up to 2.1 when the layer's stacks exceed 1
+  // GB and a second pass over them costs the most (Mixtral-shaped T = 6 (1.9) 1200 / 1324, T = 8 (2.3) 1445 /
+  // 1351, T = 128 17251 / 1814; Qwen-shaped T = 16 (1.5) 399 / 438, T = 32 (2.3) 614 / 562), up to 3 when they
+  // are under 32 MB and launches and latency set the time (d 256, d_ff 688, E 8: T = 8 (2.3) 33 / 36, T = 12
+  // (3.1) 42 / 41, T = 512 496 / 56). A dense shared expert, whose few tiles leave most CUs idle in a small
+  // batch, up to 64 rows.
   if (f32) {
     const int64_t bytes = (int64_t)E * 12 * K_in * K_out;
-    const double most = bytes < ((int64_t)32 << 20) ? 3.5 : bytes > ((int64_t)1 << 30) ? 1.8 : 2.6;
+    const double most = bytes < ((int64_t)32 << 20) ? 3.0 : bytes > ((int64_t)1 << 30) ? 2.1 : 2.6;
     return (E == 1 ? avg_m <= 64.0 : per_hit <= most) ? kGemv : kSkinny;
   }
   // packed Q4_K (the same DMA tile kernels): the GEMV up to 1.55 tokens per hit expert, then the

@@ -3,14 +3,14 @@
 // (utils.cpp:735-747) with its F32 weights; the decode GEMV (moe_experts.hip) keeps the smallest batches.
 //
 // Bound: the FP32 matrix rate (v_mfma_f32_32x32x2_f32 back to back: 155 TFLOP/s; the 16x16x4 form reaches
-// 114-137) from a few dozen rows per expert on, the weight stream below. Tiles of 64 tokens x 128 weight rows
-// (gate/up: 64 gate + 64 up, SwiGLU in the epilogue) x 32 columns, 512 threads: eight waves, 2 (M) x 4 (N), one
-// 32 x 32 subtile each. FP32 MFMAs take 64 cycles for 4 kFLOP, so LDS reads are no limit (two subtiles per
-// wave, which halve them, only cost occupancy: the sums below spilled) and the tile is chosen for balance
-// instead: small enough that ~100 rows per expert still give every CU two blocks, whose waits and epilogues
-// then overlap. Both operands go straight to LDS
-// (global_load_lds) through a ring of three stages, 16-byte granules XOR-swizzled by row pair so that the 16
-// rows a read pass touches fall on distinct bank groups.
+// 114-137) from a few dozen rows per expert on, the weight stream below. Tiles of 64 tokens x 64 weight rows
+// (gate/up: 32 gate + 32 up, SwiGLU in the epilogue) x 32 columns, 256 threads: four waves, 2 (M) x 2 (N), one
+// 32 x 32 subtile each. FP32 MFMAs take 64 cycles for 4 kFLOP, so neither LDS reads nor the L2 limit so small a
+// tile, and it is chosen for balance and registers: ~100 rows per expert give every CU several blocks, three
+// at a time, whose waits and epilogues overlap, and the sums below stay in registers (eight waves of a 128-row
+// tile, at 128 registers each, spilled, and a reload waits for all the DMA in flight). Both operands go
+// straight to LDS (global_load_lds) through a ring of three stages, 16-byte granules XOR-swizzled by row pair
+// so that the 16 rows a read pass touches fall on distinct bank groups.
 //
 // Rounding: an FP32 MFMA is a chain of FMAs, and one chain over all of K drifts with the square root of K,
 // which the GEMV's lane-parallel sums do not. So a chain runs over 8 columns only (as the GEMV's do), the eight
@@ -31,11 +31,11 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __attribute__((address_space(3))) void lds_void_f32_t;
 
-constexpr int kF32BM = 64, kF32BK = 32, kF32Rows = 128;  // tokens, columns, weight rows of a tile
-constexpr int kF32Threads = 512, kF32Stages = 3;
+constexpr int kF32BM = 64, kF32BK = 32, kF32Rows = 64;  // tokens, columns, weight rows of a tile
+constexpr int kF32Threads = 256, kF32Stages = 3;
 constexpr int kF32A = kF32BM * kF32BK * 4, kF32B = kF32Rows * kF32BK * 4;  // bytes per stage
 constexpr size_t kF32Lds = (size_t)kF32Stages * (kF32A + kF32B);
-constexpr int kF32InstA = kF32A / 1024 / 8, kF32InstB = kF32B / 1024 / 8;  // 1 KiB loads per wave and stage
+constexpr int kF32InstA = kF32A / 1024 / 4, kF32InstB = kF32B / 1024 / 4;  // 1 KiB loads per wave and stage
 constexpr int kF32Group = 4;  // m-tiles that take one n-tile's weights one after another
 
 __device__ const float4 kF32Zero = {0.0f, 0.0f, 0.0f, 0.0f};  // what columns past K load
@@ -47,8 +47,8 @@ __device__ inline void wait_vmcnt_f32() {
 }
 
 template <bool GATED>
-__global__ void __launch_bounds__(kF32Threads, 4) gemm_f32_kernel(GemmF32Args g, int NT) {
-  constexpr int BN = GATED ? 64 : 128;
+__global__ void __launch_bounds__(kF32Threads, 3) gemm_f32_kernel(GemmF32Args g, int NT) {
+  constexpr int BN = GATED ? 32 : 64;
   extern __shared__ __align__(16) uint8_t fsm[];
 
   // block -> (m-tile, n-tile, K part): the W work items in 8 equal runs, one per XCD (block b runs on XCD
@@ -76,9 +76,7 @@ __global__ void __launch_bounds__(kF32Threads, 4) gemm_f32_kernel(GemmF32Args g,
   const int kt0 = ks * nk_all / KS, nk = (ks + 1) * nk_all / KS - kt0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // (wave w runs on SIMD w % 4: each SIMD holds one wave of either M half, of which a tile of at most 32
-  // tokens idles the second)
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave >> 1, wn = wave & 1;
   const int li = lane & 31, lh = lane >> 5;
 
   // DMA sources: load j of a wave fills granules 64 (n w + j) + lane; granule gi is row gi / 8, slot gi % 8,
@@ -99,12 +97,12 @@ __global__ void __launch_bounds__(kF32Threads, 4) gemm_f32_kernel(GemmF32Args g,
   for (int i = 0; i < kF32InstB; ++i) {
     const int gi = 64 * (kF32InstB * wave + i) + lane, r = gi >> 3;
     colB[i] = 4 * ((gi & 7) ^ ((r >> 1) & 7));
-    const bool up = GATED && kF32InstB * wave + i >= 8;
+    const bool up = GATED && kF32InstB * wave + i >= 4;
     baseB[i] = (up ? g.W1 : g.W0) + ((int64_t)e * N + n0) * K;
-    offB[i] = (uint32_t)min(GATED ? (r & 63) : r, N - 1 - n0) * (uint32_t)K + (uint32_t)colB[i];
+    offB[i] = (uint32_t)min(GATED ? (r & 31) : r, N - 1 - n0) * (uint32_t)K + (uint32_t)colB[i];
   }
   // tile kt of this part; columns past its end (the last tile of K, and the tile that rounds the part up to
-  // pairs) come from a block of zeros. NOA: a wave whose activation rows (8 w .. 8 w + 7) lie past the
+  // pairs) come from a block of zeros. NOA: a wave whose activation rows (16 w .. 16 w + 15) lie past the
   // tile's tokens loads none.
   const int kend = min(K, (kt0 + nk) * kF32BK);
   auto dma = [&](const float* p, uint8_t* dst) { __builtin_amdgcn_global_load_lds(p, (lds_void_f32_t*)dst, 16, 0, 0); };
@@ -129,7 +127,7 @@ __global__ void __launch_bounds__(kF32Threads, 4) gemm_f32_kernel(GemmF32Args g,
   floatx16 sum = zero, comp = zero, mid = zero, c0 = zero, c1 = zero;
 
   // this lane's weight row in the tile; gated: the subtile's columns 0 .. 15 are gate rows, 16 .. 31 the up rows
-  const int brow = GATED ? 64 * (li >> 4) + 16 * wn + (li & 15) : 32 * wn + li;
+  const int brow = GATED ? 32 * (li >> 4) + 16 * wn + (li & 15) : 32 * wn + li;
   // columns 8 t .. 8 t + 7 of the tile: lane half lh holds 4 lh .. + 3 of them, one per MFMA, in A and B alike
   struct Frags {
     floatx4 a, b;
@@ -178,7 +176,7 @@ __global__ void __launch_bounds__(kF32Threads, 4) gemm_f32_kernel(GemmF32Args g,
     int cur = 0, fill = 2;
     if constexpr (work) load(0, 0, f0);
     // (the scheduling barriers keep the compiler from running chains ahead of the additions: their results
-    // would not fit the 128 registers of four waves per SIMD)
+    // would not fit the registers of three waves per SIMD)
     auto step = [] { __builtin_amdgcn_sched_barrier(0); };
     auto tile = [&](int kt, bool first) {
       if constexpr (work) {
@@ -218,8 +216,8 @@ __global__ void __launch_bounds__(kF32Threads, 4) gemm_f32_kernel(GemmF32Args g,
   };
   using Yes = std::integral_constant<bool, true>;
   using No = std::integral_constant<bool, false>;
-  const bool noa = 8 * wave >= rows;
-  const bool idle = 32 * wm >= rows;  // (wave >= 4, so its activation rows lie past the tokens too)
+  const bool noa = 16 * wave >= rows;
+  const bool idle = 32 * wm >= rows;  // (wave >= 2, so its activation rows lie past the tokens too)
   if (K % kF32BK == 0 && nk % 2 == 0) {
     if (idle) k_loop(Yes{}, Yes{}, Yes{});
     else if (noa) k_loop(No{}, Yes{}, Yes{});
@@ -247,15 +245,15 @@ __global__ void __launch_bounds__(kF32Threads, 4) gemm_f32_kernel(GemmF32Args g,
 }
 
 int gemm_f32_ksplit(int mtiles, int N, int K) {
-  // parts until every CU has two blocks, each part at least 8 tiles of 32 columns
+  // parts until every CU has three blocks, each part at least 8 tiles of 32 columns
   const int nt = (N + kF32Rows - 1) / kF32Rows, nk = (K + kF32BK - 1) / kF32BK;
   int ks = 1;
-  while (2 * ks <= kMaxKSplit && (int64_t)mtiles * nt * ks < 2 * std::max(1, device_cus()) && nk >= 16 * ks) ks *= 2;
+  while (2 * ks <= kMaxKSplit && (int64_t)mtiles * nt * ks < 3 * std::max(1, device_cus()) && nk >= 16 * ks) ks *= 2;
   return ks;
 }
 
 int launch_gemm_f32(const GemmF32Args& g, bool gated, int max_mtiles, hipStream_t st) {
-  const int BN = gated ? 64 : 128, NT = (g.N + BN - 1) / BN;
+  const int BN = gated ? 32 : 64, NT = (g.N + BN - 1) / BN;
   if (max_mtiles <= 0 || NT == 0) return EMBER_OK;
   static const bool ok =
       hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_kernel<true>),
