@@ -1026,11 +1026,12 @@ int launch_projection(const ProjArgs& a, hipStream_t st) {
 template <int FMT>
 struct PackRow;
 template <>
-struct PackRow<EMBER_TYPE_Q8_0> {  // the two Q8_0 blocks as they are: Fmt<Q8_0>'s chunk
+struct PackRow<EMBER_TYPE_Q8_0> {  // {dA, dB} fp16, then the blocks' quants + 128
   static constexpr int NW = 17, RB = kPackRowB;
   __device__ static void load(const uint8_t* p, uint32_t* raw) { Fmt<EMBER_TYPE_Q8_0>::load(p, 0, 0, raw); }
+  // Fmt<Q8_0>'s chunk dot: the same integers, scales and float operations
   __device__ static void dot(const uint32_t* raw, const uint8_t* x, int c, int K, float& acc) {
-    Fmt<EMBER_TYPE_Q8_0>::dot_tokens<1>(raw, x, 0, c, K, 1, &acc);
+    Fmt<EMBER_TYPE_Q8_0>::dot_tokens<1, true>(raw, x, 0, c, K, 1, &acc);
   }
 };
 template <>

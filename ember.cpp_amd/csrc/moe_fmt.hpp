@@ -148,11 +148,12 @@ struct Fmt<EMBER_TYPE_Q8_0> {
   }
   // MT tokens' dots of one chunk; the activation rows are staged in LDS (act_lds_bytes layout).
   // Each weight pair is converted once (q + 128, zero-extended to 16 bits) and used for every token.
-  template <int MT>
+  // PACK: raw is a prefill pack row ({dA, dB}, then the two blocks' q + 128).
+  template <int MT, bool PACK = false>
   __device__ static void dot_tokens(const uint32_t* raw, const uint8_t* lds, int row_lds, int c, int K, int nvalid,
                                     float* out) {
     const float dA = half_bits_to_float(raw[0] & 0xffff);
-    const float dB = half_bits_to_float(raw[8] >> 16);
+    const float dB = half_bits_to_float((PACK ? raw[0] : raw[8]) >> 16);
     int ia[MT], ib[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) ia[m] = ib[m] = 0;
@@ -161,8 +162,9 @@ struct Fmt<EMBER_TYPE_Q8_0> {
       uint32_t ua[4], ub[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        ua[j] = u16pair(raw[(1 + j4 + j) >> 1] ^ 0x80808080u, (1 + j4 + j) & 1);
-        ub[j] = u16pair(raw[9 + ((j4 + j) >> 1)] ^ 0x80808080u, (j4 + j) & 1);
+        ua[j] = PACK ? u16pair(raw[1 + ((j4 + j) >> 1)], (j4 + j) & 1)
+                     : u16pair(raw[(1 + j4 + j) >> 1] ^ 0x80808080u, (1 + j4 + j) & 1);
+        ub[j] = u16pair(raw[9 + ((j4 + j) >> 1)] ^ (PACK ? 0u : 0x80808080u), (j4 + j) & 1);
       }
 #pragma unroll
       for (int m = 0; m < MT; ++m) {

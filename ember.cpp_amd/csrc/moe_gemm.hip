@@ -32,6 +32,7 @@ typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
 
 constexpr int GBM = 256, GBK = 64, LDK = GBK + 8;  // LDS rows padded by 16 bytes
@@ -522,22 +523,67 @@ struct DmaW {
 };
 
 // The B fragment of K step KS (compile time) from one weight row's K tile in LDS: the lane's 8 elements
-// of K granule 2 KS + h, as fp16 MFMA operands.
-// Q8_0: K granule gk = 2 ks + h of the 64 = Q8_0 block b = ks / 2, bytes X + 8 h .. + 8 of the row's 68
-// with X = 34 b + 2 + 16 (ks % 2); for b = 1 those are dword aligned and, in row slices past byte 52,
-// read from the overlapping fifth granule (LDS byte = global byte + 12); for b = 0 they sit two bytes
-// past a dword and are funnel-shifted out of three dwords. Value d * q, one rounding.
+// of K granule 2 KS + h, as fp16 MFMA operands; in two halves, so that a kernel can let MFMAs run between the LDS
+// reads (load_b) and the decode of what they return (decode_b). A raw fragment is kept over a tile's K steps
+// (0, 1, 2, 3 in order): a step reads only what the steps before it have not.
+// Q8_0 rows: K granule gk = 2 ks + h of the 64 = Q8_0 block b = ks / 2, bytes X + 8 h .. + 8 of the row's 68
+// with X = 34 b + 2 + 16 (ks % 2); for b = 1 those are dword aligned and, past byte 52, read from the
+// overlapping fifth granule (LDS byte = global byte + 12); for b = 0 they sit two bytes past a dword and
+// are funnel-shifted out of three dwords. Value d * q, one rounding.
+// Q8_0 pack: the two blocks' d, then their 64 quants + 128 in order: both dwords aligned. The same values.
 // Q4_K pack: group b = ks / 2 (its nibble half of the 32 bytes), elements 16 (ks % 2) + 8 h .. + 8 =
-// nibble bytes of the same offsets; value a * q + m by one fp16 fused multiply-add (the factors as
-// Deq<Q4_K> forms them, so the products are those of the register-staged kernels).
+// nibble bytes of the same offsets (steps 2 and 3 take the high nibbles of what 0 and 1 read); value a * q + m
+// by one fp16 fused multiply-add (the factors as Deq<Q4_K> forms them, so the products are those of the
+// register-staged kernels).
+template <int WF>
+struct RawB {
+  uint32_t hdr[2];   // packs: the row's scale factors; rows: hdr[0] the dword that holds the block's d
+  uint32_t w[2][3];  // quants of the K step (Q4_K pack: of steps 0 and 1)
+};
 template <int WF, int KS>
-__device__ inline half8 b_frag(const uint8_t* row, int h) {
+__device__ inline void load_b(const uint8_t* row, int h, RawB<WF>& r) {
+  if constexpr (WF == kWfQ4Pack) {
+    if constexpr (KS == 0) {
+      const u32x2 v = *reinterpret_cast<const u32x2*>(row);
+      r.hdr[0] = v.x;
+      r.hdr[1] = v.y;
+    }
+    if constexpr (KS < 2) {
+      const u32x2 v = *reinterpret_cast<const u32x2*>(row + 8 + 16 * KS + 8 * h);
+      r.w[KS][0] = v.x;
+      r.w[KS][1] = v.y;
+    }
+  } else if constexpr (WF == kWfQ8Pack) {
+    const uint32_t* qw = reinterpret_cast<const uint32_t*>(row + 4 + 16 * KS + 8 * h);
+    r.w[0][0] = qw[0];
+    r.w[0][1] = qw[1];
+    if constexpr (KS == 0) r.hdr[0] = *reinterpret_cast<const uint32_t*>(row);
+  } else {
+    constexpr int b = KS >> 1, X = 34 * b + 2 + 16 * (KS & 1);
+    if constexpr (b == 0) {
+      const uint32_t* qw = reinterpret_cast<const uint32_t*>(row + (X & ~3) + 8 * h);
+      r.w[0][0] = qw[0];
+      r.w[0][1] = qw[1];
+      r.w[0][2] = qw[2];
+    } else {
+      const int byte = X + 8 * h;
+      const uint32_t* qw = reinterpret_cast<const uint32_t*>(row + (byte + 8 <= 64 ? byte : byte + 12));
+      r.w[0][0] = qw[0];
+      r.w[0][1] = qw[1];
+    }
+    if constexpr ((KS & 1) == 0) r.hdr[0] = *reinterpret_cast<const uint32_t*>(row + 32 * b);
+  }
+}
+template <int HI>
+__device__ inline half2_t both(uint32_t v) {  // one half of v in both halves (an operand select, no instruction)
+  return __builtin_shufflevector(h2(v), h2(v), HI, HI);
+}
+template <int WF, int KS>
+__device__ inline half8 decode_b(const RawB<WF>& r) {
   constexpr int b = KS >> 1;
   if constexpr (WF == kWfQ4Pack) {
-    const uint32_t hdr = *reinterpret_cast<const uint32_t*>(row + 4 * b);
-    const half2_t a = h2((hdr & 0xffffu) * 0x10001u), m = h2((hdr >> 16) * 0x10001u);
-    const uint32_t* qw = reinterpret_cast<const uint32_t*>(row + 8 + 16 * (KS & 1) + 8 * h);
-    const uint32_t n0 = (qw[0] >> (4 * b)) & 0x0f0f0f0fu, n1 = (qw[1] >> (4 * b)) & 0x0f0f0f0fu;
+    const half2_t a = both<0>(r.hdr[b]), m = both<1>(r.hdr[b]);
+    const uint32_t n0 = (r.w[KS & 1][0] >> (4 * b)) & 0x0f0f0f0fu, n1 = (r.w[KS & 1][1] >> (4 * b)) & 0x0f0f0f0fu;
     const half2_t off = h2(0xe400e400u);  // -1024 in each half
     const uint32_t o0 = u32(__builtin_elementwise_fma(magic_pair(n0, 0) + off, a, m));
     const uint32_t o1 = u32(__builtin_elementwise_fma(magic_pair(n0, 1) + off, a, m));
@@ -545,24 +591,18 @@ __device__ inline half8 b_frag(const uint8_t* row, int h) {
     const uint32_t o3 = u32(__builtin_elementwise_fma(magic_pair(n1, 1) + off, a, m));
     return __builtin_bit_cast(half8, u32x4{o0, o1, o2, o3});
   } else {
-    constexpr int X = 34 * b + 2 + 16 * (KS & 1);
-    const uint32_t dbits = b ? (*reinterpret_cast<const uint32_t*>(row + 32) >> 16)
-                             : (*reinterpret_cast<const uint32_t*>(row) & 0xffffu);
-    const half2_t d = h2(dbits * 0x10001u);
-    uint32_t w0, w1;
-    if constexpr (b == 0) {
-      const uint32_t* qw = reinterpret_cast<const uint32_t*>(row + (X & ~3) + 8 * h);
-      w0 = __builtin_amdgcn_alignbit(qw[1], qw[0], 16);
-      w1 = __builtin_amdgcn_alignbit(qw[2], qw[1], 16);
+    uint32_t q0, q1;
+    half2_t d;
+    if constexpr (WF == kWfQ8Pack) {
+      q0 = r.w[0][0];
+      q1 = r.w[0][1];
+      d = both<b>(r.hdr[0]);
     } else {
-      const int byte = X + 8 * h;
-      const uint32_t* qw =
-          reinterpret_cast<const uint32_t*>(row + (WF == kWfQ8Pack || byte + 8 <= 64 ? byte : byte + 12));
-      w0 = qw[0];
-      w1 = qw[1];
+      q0 = (b == 0 ? __builtin_amdgcn_alignbit(r.w[0][1], r.w[0][0], 16) : r.w[0][0]) ^ 0x80808080u;
+      q1 = (b == 0 ? __builtin_amdgcn_alignbit(r.w[0][2], r.w[0][1], 16) : r.w[0][1]) ^ 0x80808080u;
+      d = both<b>(r.hdr[0]);
     }
     const half2_t off = h2(0xe480e480u);  // -1152 = -(1024 + 128) in each half
-    const uint32_t q0 = w0 ^ 0x80808080u, q1 = w1 ^ 0x80808080u;
     const uint32_t o0 = u32((magic_pair(q0, 0) + off) * d), o1 = u32((magic_pair(q0, 1) + off) * d);
     const uint32_t o2 = u32((magic_pair(q1, 0) + off) * d), o3 = u32((magic_pair(q1, 1) + off) * d);
     return __builtin_bit_cast(half8, u32x4{o0, o1, o2, o3});
@@ -648,24 +688,20 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_q8_kernel(GemmArgs g, in
                 (part < 4 ? 16 * part : 52);
     }
   }
-  // DMA of tile kt (clamped: tiles past the end reload the last, never multiplied), part j of 4 so
-  // that the issue is spread over the K steps of a tile: activation instruction j, weight instruction j
+  // DMA of tile kt (clamped: tiles past the end reload the last, never multiplied) into the stage at byte
+  // `st`, part j of 4 so that the issue is spread over the K steps of a tile: activation instruction j, weight
+  // instruction j
   // NOA (compile time): this wave loads no activation rows (its rows lie past the tile's tokens), so its
   // per-tile DMA count, and the waits that count it, are the weights' alone
-  auto issue = [&](int kt, int j, auto NOAc) {
+  auto issue = [&](int kt, int st, int j, auto NOAc) {
     const int kc = kt0 + min(kt, nk - 1);
-    uint8_t* st = dsm + (kt % NS) * kStage;
     if constexpr (!decltype(NOAc)::value) {
       if (j < kInstA)
-        lds_dma16(srcA[j < kInstA ? j : 0] + (size_t)kc * GBK * 2, st + 1024 * (kInstA * wave + j));
+        lds_dma16(srcA[j < kInstA ? j : 0] + (size_t)kc * GBK * 2, dsm + st + 1024 * (kInstA * wave + j));
     }
     if (j < kDmaInstB)
       lds_dma16(srcB[j < kDmaInstB ? j : 0] + (size_t)kc * DmaW<WF>::kStride,
-                st + kAB + 1024 * min(kDmaInstB * wave + j, kLastB));
-  };
-  auto issue_all = [&](int kt, auto NOAc) {
-#pragma unroll
-    for (int j = 0; j < kInstMax; ++j) issue(kt, j, NOAc);
+                dsm + st + kAB + 1024 * min(kDmaInstB * wave + j, kLastB));
   };
 
   floatx16 acc[4][2];
@@ -676,38 +712,15 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_q8_kernel(GemmArgs g, in
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][jn][r] = 0.0f;
 
-  // B tile row of this lane in subtile jn
-  auto brow_of = [&](int jn) {
-    if constexpr (GATED) return jn * 128 + wn * 32 + (lane & 31);
-    return wn * 64 + 32 * jn + (lane & 31);
-  };
-  const int h = lane >> 5;
+  const int h = lane >> 5, li = lane & 31;
+  // This lane's LDS bytes within a stage: its activation row of subtile 0 at K step ks (subtile i 4 KiB on; the
+  // swizzle is the same for rows a multiple of 16 apart) and its weight row of subtile jn
+  uint32_t offA[4], offB[2];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) offA[ks] = 128 * (wm * 128 + li) + 16 * ((2 * ks + h) ^ ((li >> 1) & 7));
+#pragma unroll
+  for (int jn = 0; jn < 2; ++jn) offB[jn] = kAB + kRowB * (GATED ? jn * 128 + wn * 32 + li : wn * 64 + 32 * jn + li);
 
-  // Fragments of K step ks (compile time) of the tile in stage `st`, for the first MS (compile time)
-  // 32-row subtiles
-  struct Frags {
-    half8 a[4], b[2];
-  };
-  auto load_frags = [&](const uint8_t* st, auto KS, auto MSc, Frags& f) {
-    constexpr int ks = decltype(KS)::value;
-    constexpr int MS = decltype(MSc)::value;
-    const int gk = 2 * ks + h;
-#pragma unroll
-    for (int i = 0; i < MS; ++i) {
-      const int r = wm * 128 + 32 * i + (lane & 31);
-      f.a[i] = *reinterpret_cast<const half8*>(st + 16 * (8 * r + (gk ^ ((r >> 1) & 7))));
-    }
-    const uint8_t* Bs = st + kAB;
-#pragma unroll
-    for (int jn = 0; jn < 2; ++jn) f.b[jn] = b_frag<WF, ks>(Bs + kRowB * brow_of(jn), h);
-  };
-  auto mfmas = [&](const Frags& f, auto MSc) {
-#pragma unroll
-    for (int i = 0; i < decltype(MSc)::value; ++i)
-#pragma unroll
-      for (int jn = 0; jn < 2; ++jn)
-        acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(f.a[i], f.b[jn], acc[i][jn], 0, 0, 0);
-  };
   // A bare barrier: __syncthreads()'s release fence would wait for the DMA in flight as well. The
   // empty asm statements keep the compiler from moving LDS accesses across it.
   auto barrier = [] {
@@ -723,41 +736,87 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_q8_kernel(GemmArgs g, in
   // A wave whose M half holds no tokens (MS = 0) only loads and keeps the barriers.
   // (NS stages: tiles kt + 1 .. kt + NS - 2 are in flight while tile kt is multiplied; the iteration
   // issues tile kt + NS - 1 and then waits for tile kt + 1, leaving NS - 2 tiles' DMA outstanding)
-  auto k_loop = [&](auto MSc, auto NOAc) {
+  // Each step is written as the next step's LDS reads, its own MFMAs, then the next step's decode. ORD (compile
+  // time): a scheduling barrier keeps the compiler from mixing steps, for full subtiles of both M halves, where
+  // two waves per SIMD cover each other's reads (Mixtral-shaped Q8_0 T = 2048 1848 -> 1791 us, Qwen-shaped Q4_K
+  // T = 4096 662 -> 649); where the second half holds no tokens it is better off hoisting reads across steps
+  // (Mixtral-shaped Q4_K T = 512 547 us, 565 with the barrier). Finer orders (scheduling groups: reads first, one
+  // MFMA per 4 to 6 decode instructions) were slower than either.
+  auto k_loop = [&](auto MSc, auto NOAc, auto ORDc) {
+    constexpr int MS = decltype(MSc)::value;
     constexpr int kInst = decltype(NOAc)::value ? kDmaInstB : kDmaInst;  // this wave's DMA per tile
+    half8 fa[2][MS > 0 ? MS : 1], fb[2][2];
+    RawB<WF> raw[2];
+    auto read = [&](int st, auto KSc, half8 (&a)[MS > 0 ? MS : 1]) {
+      constexpr int ks = decltype(KSc)::value;
+#pragma unroll
+      for (int jn = 0; jn < 2; ++jn) load_b<WF, ks>(dsm + st + offB[jn], h, raw[jn]);
+#pragma unroll
+      for (int i = 0; i < MS; ++i) a[i] = *reinterpret_cast<const half8*>(dsm + st + offA[ks] + 4096 * i);
+    };
+    auto decode = [&](auto KSc, half8 (&b)[2]) {
+#pragma unroll
+      for (int jn = 0; jn < 2; ++jn) b[jn] = decode_b<WF, decltype(KSc)::value>(raw[jn]);
+    };
+    auto mfmas = [&](const half8 (&a)[MS > 0 ? MS : 1], const half8 (&b)[2]) {
+#pragma unroll
+      for (int i = 0; i < MS; ++i)
+#pragma unroll
+        for (int jn = 0; jn < 2; ++jn)
+          acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[jn], acc[i][jn], 0, 0, 0);
+    };
+    auto order = [] {
+      if constexpr (MS >= 4 && decltype(ORDc)::value) __builtin_amdgcn_sched_barrier(0);
+    };
     using K0 = std::integral_constant<int, 0>;
     using K1 = std::integral_constant<int, 1>;
     using K2 = std::integral_constant<int, 2>;
     using K3 = std::integral_constant<int, 3>;
 #pragma unroll
-    for (int t = 0; t < NS - 1; ++t) issue_all(t, NOAc);
+    for (int t = 0; t < NS - 1; ++t)
+#pragma unroll
+      for (int j = 0; j < kInstMax; ++j) issue(t, t * kStage, j, NOAc);
     wait_vmcnt<(NS - 2) * kInst>();
     barrier();
-    Frags f0, f1;
-    if constexpr (decltype(MSc)::value > 0) load_frags(dsm, K0{}, MSc, f0);
+    if constexpr (MS > 0) {
+      read(0, K0{}, fa[0]);
+      decode(K0{}, fb[0]);
+    }
+    int cur = 0, fill = (NS - 1) * kStage;  // the stage of tile kt and the one the iteration refills
     for (int kt = 0; kt < nk; ++kt) {
-      if constexpr (decltype(MSc)::value == 0) {
-        issue_all(kt + NS - 1, NOAc);
+      const int nxt = cur == (NS - 1) * kStage ? 0 : cur + kStage;
+      if constexpr (MS == 0) {
+#pragma unroll
+        for (int j = 0; j < kInstMax; ++j) issue(kt + NS - 1, fill, j, NOAc);
         wait_vmcnt<(NS - 2) * kInst>();
         barrier();
       } else {
-        const uint8_t* st = dsm + (kt % NS) * kStage;
-        load_frags(st, K1{}, MSc, f1);
-        issue(kt + NS - 1, 0, NOAc);
-        mfmas(f0, MSc);
-        load_frags(st, K2{}, MSc, f0);
-        issue(kt + NS - 1, 1, NOAc);
-        mfmas(f1, MSc);
-        load_frags(st, K3{}, MSc, f1);
-        issue(kt + NS - 1, 2, NOAc);
-        mfmas(f0, MSc);
-        issue(kt + NS - 1, 3, NOAc);
+        read(cur, K1{}, fa[1]);
+        issue(kt + NS - 1, fill, 0, NOAc);
+        mfmas(fa[0], fb[0]);
+        decode(K1{}, fb[1]);
+        order();
+        read(cur, K2{}, fa[0]);
+        issue(kt + NS - 1, fill, 1, NOAc);
+        mfmas(fa[1], fb[1]);
+        decode(K2{}, fb[0]);
+        order();
+        read(cur, K3{}, fa[1]);
+        issue(kt + NS - 1, fill, 2, NOAc);
+        issue(kt + NS - 1, fill, 3, NOAc);
+        mfmas(fa[0], fb[0]);
+        decode(K3{}, fb[1]);
+        order();
         wait_vmcnt<(NS - 2) * kInst>();
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of tile kt are complete
         barrier();
-        load_frags(dsm + ((kt + 1) % NS) * kStage, K0{}, MSc, f0);
-        mfmas(f1, MSc);
+        read(nxt, K0{}, fa[0]);
+        mfmas(fa[1], fb[1]);
+        decode(K0{}, fb[0]);
+        order();
       }
+      fill = cur;
+      cur = nxt;
     }
   };
   __shared__ int s_rexp[GBM];
@@ -769,21 +828,26 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_q8_kernel(GemmArgs g, in
   // (SHORT: msub <= 2, so the 3- and 4-subtile loops are not built)
   using M4 = std::integral_constant<int, SHORT ? 2 : 4>;
   using M3 = std::integral_constant<int, SHORT ? 2 : 3>;
-  if (8 * kInstA * wave >= rows) {
+  using M2 = std::integral_constant<int, 2>;
+  using M1 = std::integral_constant<int, 1>;
+  using M0 = std::integral_constant<int, 0>;
+  if (8 * kInstA * wave >= rows) {  // (four subtiles of a half fill all of its waves' activation rows)
     switch (msub) {
-      case 4: k_loop(M4{}, A0{}); break;
-      case 3: k_loop(M3{}, A0{}); break;
-      case 2: k_loop(std::integral_constant<int, 2>{}, A0{}); break;
-      case 1: k_loop(std::integral_constant<int, 1>{}, A0{}); break;
-      default: k_loop(std::integral_constant<int, 0>{}, A0{}); break;
+      case 3: k_loop(M3{}, A0{}, A1{}); break;
+      case 2: k_loop(M2{}, A0{}, A1{}); break;
+      case 1: k_loop(M1{}, A0{}, A1{}); break;
+      default: k_loop(M0{}, A0{}, A1{}); break;
     }
   } else {
     switch (msub) {
-      case 4: k_loop(M4{}, A1{}); break;
-      case 3: k_loop(M3{}, A1{}); break;
-      case 2: k_loop(std::integral_constant<int, 2>{}, A1{}); break;
-      case 1: k_loop(std::integral_constant<int, 1>{}, A1{}); break;
-      default: k_loop(std::integral_constant<int, 0>{}, A1{}); break;
+      case 4:
+        if (rows > 128) k_loop(M4{}, A1{}, A0{});
+        else k_loop(M4{}, A1{}, A1{});
+        break;
+      case 3: k_loop(M3{}, A1{}, A1{}); break;
+      case 2: k_loop(M2{}, A1{}, A1{}); break;
+      case 1: k_loop(M1{}, A1{}, A1{}); break;
+      default: k_loop(M0{}, A1{}, A1{}); break;
     }
   }
   wait_vmcnt<0>();  // no DMA may still target LDS when the block exits
@@ -918,6 +982,7 @@ __global__ void __launch_bounds__(kD64Threads) gemm_dma64_q8_kernel(GemmArgs g, 
   struct Frags {
     half8 a[2], b[2];
   };
+  RawB<WF> raw[2];
   auto load_frags = [&](const uint8_t* st, auto KS, Frags& f) {
     constexpr int ks = decltype(KS)::value;
     const int gk = 2 * ks + h;
@@ -928,7 +993,10 @@ __global__ void __launch_bounds__(kD64Threads) gemm_dma64_q8_kernel(GemmArgs g, 
     }
     const uint8_t* Bs = st + kD64A;
 #pragma unroll
-    for (int jn = 0; jn < 2; ++jn) f.b[jn] = b_frag<WF, ks>(Bs + kRowB * brow_of(jn), h);
+    for (int jn = 0; jn < 2; ++jn) {
+      load_b<WF, ks>(Bs + kRowB * brow_of(jn), h, raw[jn]);
+      f.b[jn] = decode_b<WF, ks>(raw[jn]);
+    }
   };
   auto mfmas = [&](const Frags& f) {
 #pragma unroll
@@ -1604,10 +1672,18 @@ __global__ void __launch_bounds__(256) prefill_pack_kernel(const uint8_t* __rest
 #pragma unroll
     for (int w = 0; w < 8; ++w) d[2 + w] = raw[4 + w];
   } else {
+    // (a ggml row's 68 bytes: dword 0 = {dA, q0, q1}, ..., 8 = {q30, q31, dB}, 9.. = block B)
     const uint32_t* src = reinterpret_cast<const uint32_t*>(row + (int64_t)kc * kPackRowB);
     uint32_t* d = reinterpret_cast<uint32_t*>(dst + i * kPackRowB);
+    uint32_t w[kPackRowB / 4];
 #pragma unroll
-    for (int w = 0; w < kPackRowB / 4; ++w) d[w] = src[w];
+    for (int j = 0; j < kPackRowB / 4; ++j) w[j] = src[j];
+    d[0] = (w[0] & 0xffffu) | (w[8] & 0xffff0000u);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      d[1 + j] = __builtin_amdgcn_alignbit(w[j + 1], w[j], 16) ^ 0x80808080u;
+      d[9 + j] = w[9 + j] ^ 0x80808080u;
+    }
   }
 }
 

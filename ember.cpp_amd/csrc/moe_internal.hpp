@@ -311,7 +311,8 @@ int launch_bf16_pair_max(const int16_t* ge, const int16_t* ue, int E, int N, int
 // the gate/up section [E][ceil(d_ff / 128)][d / 64] (each tile: the 128 gate rows of an n-tile, then
 // its 128 up rows), then the down section [E][ceil(d / 256)][d_ff / 64]; rows past a matrix's end
 // repeat its last row (as the GEMM's clamped loads would). A row's 64 columns:
-//   Q8_0 stacks: the two Q8_0 blocks as they are (68 bytes);
+//   Q8_0 stacks: 68 bytes = the fp16 scales {dA, dB} of its two blocks, then their 64 quants + 128 (dword
+//     aligned and unsigned, as the tile kernels' and the one-token slices' decoders take them);
 //   Q4_K stacks: 40 bytes = the fp16 factors {a0, m0, a1, m1} of its two 32-element groups, a = d * sc
 //     and m = -dmin * mn each rounded to fp16 once (weight = a * q + m), then the 32 nibble bytes of the
 //     super-block quarter as they are (low nibbles: group 0, high nibbles: group 1).
