@@ -290,7 +290,7 @@ Layout layout(const ember_moe_layer* w, int T) {
   l.hexp = o; o = align_up(o + (mfma && !sp ? slots * 4 : 0));
   l.hs16 = o; o = align_up(o + (mfma_sh ? (size_t)T * w->d_ff_shared * (sp_sh ? 4 : 2) : 0));
   l.hsexp = o; o = align_up(o + (mfma_sh && !sp_sh ? (size_t)T * 4 : 0));
-  l.tiles = o; o = align_up(o + tiles * 8);
+  l.tiles = o; o = align_up(o + tiles * 16);
   // the routed gate/up's tail split (256-token tiles): raw partial gate / up dots [parts][T k][2 d_ff]
   l.tail_parts = l.mode == kGemm ? gemm_tail_parts(w->gate_type, w->prefill_pack != nullptr && !pack_bf16,
                                                    (int)slots, w->d_ff, w->d)
@@ -346,7 +346,8 @@ DispatchScratch dispatch_scratch(void* scratch, const RouteLayout& r, int32_t* o
   ds.n_used = at<int32_t>(scratch, r.n_used);
   ds.perm = perm;
   ds.pos = at<int32_t>(scratch, r.pos);
-  ds.tiles = ds.n_tiles = nullptr;
+  ds.tiles = nullptr;
+  ds.n_tiles = nullptr;
   ds.tile_bm = 0;
   return ds;
 }
@@ -466,7 +467,7 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
   int32_t* perm = at<int32_t>(scratch, l.perm);
   DispatchScratch ds = dispatch_scratch(scratch, l.r, offsets, perm);
   if (l.mode != kGemv) {  // the dispatch also writes the MFMA GEMMs' tile table
-    ds.tiles = at<int32_t>(scratch, l.tiles);
+    ds.tiles = at<int4>(scratch, l.tiles);
     ds.n_tiles = at<int32_t>(scratch, l.n_tiles);
     ds.tile_bm = gemm_tile_rows(l.mode == kSkinny);
   }
@@ -653,7 +654,6 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     g.K = d;
     g.tiles = ds.tiles;
     g.n_tiles = ds.n_tiles;
-    g.offsets = offsets;
     g.out = h;
     g.ksplit = 1;
     const int mt = gemm_skinny_max_tiles(T, k, E);
@@ -675,7 +675,7 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     auto gemm = [&](const GemmArgs& g, bool gated, int mt) {
       return skinny ? launch_gemm_skinny(g, gated, mt, st) : launch_gemm(g, gated, mt, st);
     };
-    int32_t* tiles = ds.tiles;
+    const int4* tiles = ds.tiles;
     int32_t* n_tiles = ds.n_tiles;
     _Float16* h16 = at<_Float16>(scratch, l.h16);
     int32_t* hexp = at<int32_t>(scratch, l.hexp);
@@ -698,7 +698,6 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     g.K = d;
     g.tiles = tiles;
     g.n_tiles = n_tiles;
-    g.offsets = offsets;
     g.out_h = h16;
     // the prefill pack serves the DMA tile kernels (256- and 64-token tiles alike)
     const PackLayout pl = pack_layout(d, d_ff, E, w->gate_type);

@@ -248,6 +248,21 @@ __device__ inline void load_row_exps(const GemmArgs& g, int p0, int rows, int* s
   for (int r = threadIdx.x; r < rows; r += blockDim.x) s_rexp[r] = row_exp(g, p0 + r);
 }
 
+// Row tile mt of a launch of bm-token tiles: expert e (0 for dense rows), first position p0 and rows (0: none)
+__device__ inline void row_tile(const GemmArgs& g, int mt, int bm, int& e, int& p0, int& rows) {
+  if (g.tiles) {
+    const int4 t = g.tiles[mt];
+    e = t.x;
+    p0 = t.y;
+    rows = t.z;
+  } else {
+    const int h = tile_height(g.T, bm);
+    e = 0;
+    p0 = mt * h;
+    rows = max(0, min(h, g.T - p0));
+  }
+}
+
 // m-tiles of a launch: the device-side tile count, or the dense rows' tiles of bm tokens
 __device__ inline int launch_mtiles(const GemmArgs& g, int bm) {
   return g.tiles ? *g.n_tiles : (g.T + bm - 1) / bm;
@@ -333,17 +348,9 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
   // ---- the tile
   int mt, nt;
   if (!xcd_item(launch_mtiles(g, GBM), NT, 1, mt, nt)) return;
-  int e = 0, p0 = 0, rows = 0;
-  if (g.tiles) {
-    e = g.tiles[2 * mt];
-    const int m0 = g.tiles[2 * mt + 1];
-    p0 = g.offsets[e] + m0;
-    rows = min(GBM, g.offsets[e + 1] - p0);
-  } else {
-    p0 = mt * GBM;
-    if (p0 >= g.T) return;
-    rows = min(GBM, g.T - p0);
-  }
+  int e, p0, rows;
+  row_tile(g, mt, GBM, e, p0, rows);
+  if (rows <= 0) return;
   const int n0 = nt * BN;
   const int K = g.K, N = g.N;
   const int nk = K / GBK;
@@ -636,17 +643,9 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_q8_kernel(GemmArgs g, in
     nt = rem / KS;
     ks = rem % KS;
   }
-  int e = 0, p0 = 0, rows = 0;
-  if (g.tiles) {
-    e = g.tiles[2 * mt];
-    const int m0 = g.tiles[2 * mt + 1];
-    p0 = g.offsets[e] + m0;
-    rows = min(GBM, g.offsets[e + 1] - p0);
-  } else {
-    p0 = mt * GBM;
-    if (p0 >= g.T) return;
-    rows = min(GBM, g.T - p0);
-  }
+  int e, p0, rows;
+  row_tile(g, mt, GBM, e, p0, rows);
+  if (rows <= 0) return;
   const int n0 = nt * BN;
   const int K = g.K, N = g.N;
   // this part's K tiles [kt0, kt0 + nk)
@@ -909,17 +908,9 @@ __global__ void __launch_bounds__(kD64Threads) gemm_dma64_q8_kernel(GemmArgs g, 
   if ((int)blockIdx.x >= M * NT * (g.ksplit < 1 ? 1 : g.ksplit)) return;
   const int mt = blockIdx.x % M, rest = blockIdx.x / M;
   const int nt = rest % NT, ks = rest / NT;
-  int e = 0, p0 = 0, rows = 0;
-  if (g.tiles) {
-    e = g.tiles[2 * mt];
-    const int m0 = g.tiles[2 * mt + 1];
-    p0 = g.offsets[e] + m0;
-    rows = min(kD64BM, g.offsets[e + 1] - p0);
-  } else {
-    p0 = mt * kD64BM;
-    if (p0 >= g.T) return;
-    rows = min(kD64BM, g.T - p0);
-  }
+  int e, p0, rows;
+  row_tile(g, mt, kD64BM, e, p0, rows);
+  if (rows <= 0) return;
   const int n0 = nt * BN;
   const int K = g.K, N = g.N;
   const int nk_all = K / GBK;
@@ -1099,17 +1090,9 @@ __global__ void __launch_bounds__(256) gemm_skinny_kernel(GemmArgs g, int NT) {
   const int mt = blockIdx.x % M, rest = blockIdx.x / M;
   const int nt = rest % NT, ks = rest / NT;
   const int KS = g.ksplit < 1 ? 1 : g.ksplit;
-  int e = 0, p0 = 0, rows = 0;
-  if (g.tiles) {
-    e = g.tiles[2 * mt];
-    const int m0 = g.tiles[2 * mt + 1];
-    p0 = g.offsets[e] + m0;
-    rows = min(SBM, g.offsets[e + 1] - p0);
-  } else {
-    p0 = mt * SBM;
-    if (p0 >= g.T) return;
-    rows = min(SBM, g.T - p0);
-  }
+  int e, p0, rows;
+  row_tile(g, mt, SBM, e, p0, rows);
+  if (rows <= 0) return;
   const int K = g.K, N = g.N, nk_all = K / GBK;
   const int kt0 = ks * nk_all / KS, nk = (ks + 1) * nk_all / KS - kt0;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1312,8 +1295,8 @@ __global__ void __launch_bounds__(256) gemm_tail_fixup_kernel(GemmArgs g, int NT
   const int S = tail_split(g, W, full);
   if (S <= 1 || (int)blockIdx.x >= W - full) return;
   const int w = full + blockIdx.x, mt = w / NT, nt = w % NT;
-  const int e = g.tiles[2 * mt], m0 = g.tiles[2 * mt + 1];
-  const int p0 = g.offsets[e] + m0, rows = min(GBM, g.offsets[e + 1] - p0);
+  int e, p0, rows;
+  row_tile(g, mt, GBM, e, p0, rows);
   const int N = g.N, n0 = nt * BN;
   const size_t stride = (size_t)g.part_rows * 2 * N;
   for (int i = threadIdx.x; i < rows * BN; i += 256) {

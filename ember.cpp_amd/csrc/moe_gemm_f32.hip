@@ -63,13 +63,17 @@ __global__ void __launch_bounds__(kF32Threads, 3) gemm_f32_kernel(GemmF32Args g,
   const int rest = w / kF32Group % (NT * KS);
   const int nt = rest / KS, ks = rest % KS;
   if (mt >= M) return;
-  int e = 0, p0 = mt * kF32BM, end = g.T;
+  int e = 0, p0, rows;
   if (g.tiles) {
-    e = g.tiles[2 * mt];
-    p0 = g.offsets[e] + g.tiles[2 * mt + 1];
-    end = g.offsets[e + 1];
+    const int4 t = g.tiles[mt];
+    e = t.x;
+    p0 = t.y;
+    rows = t.z;
+  } else {
+    const int h = tile_height(g.T, kF32BM);
+    p0 = mt * h;
+    rows = min(h, g.T - p0);
   }
-  const int rows = min(kF32BM, end - p0);
   if (rows <= 0) return;
   const int n0 = nt * BN, K = g.K, N = g.N;
   const int nk_all = (K + kF32BK - 1) / kF32BK;

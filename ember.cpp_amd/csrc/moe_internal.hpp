@@ -28,6 +28,18 @@ __device__ inline void copy16_to_lds(void* dst, const void* src, int n) {
   }
 }
 
+// Rows of one tile of a segment of n rows, for tiles of at most bm (a multiple of 32): whole tiles, or, when the
+// last of them would hold more than 32 rows but not all, as many of equal height in 32-row steps (n = 300, bm =
+// 256: 160 + 140 rows). A 256-token tile's time follows its 32-row steps, so equal tiles keep the CUs level
+// (Mixtral-shaped, whole / equal tiles: Q8_0 T = 1200, ~300 rows per expert, 1103 / 1062 us, Q4_K T = 1400 1107 /
+// 1071); a tile of one step costs little more than streaming its weights, so few rows past whole tiles
+// stay in one (Qwen-shaped T = 4096, 256 rows per expert and a few, 632 / 638 us, Mixtral-shaped T = 2048 1721 /
+// 1727).
+__host__ __device__ inline int tile_height(int n, int bm) {
+  const int nt = (n + bm - 1) / bm;
+  return nt <= 1 || n - (nt - 1) * bm <= 32 ? bm : ((n + nt - 1) / nt + 31) / 32 * 32;
+}
+
 // Device buffers of the dispatch step, carved from the caller's scratch.
 // Activation conversion for the MFMA paths (act_conv_row): x [rows][K] f32 into fp16 rows scaled by 2^-e
 // (y16, e in yexp; null: not needed) and / or split bf16 planes (yb, lo plane `plane` elements on; null:
@@ -50,8 +62,9 @@ struct DispatchScratch {
   int32_t* perm;       // [T*k] sorted position -> slot t*k+j
   int32_t* pos;        // [T*k] slot -> sorted position (-1: no pick)
   // optional (null: none): the MFMA GEMMs' tile table, written by the dispatch's last step: tiles of
-  // tile_bm rows over each expert's segment, experts ascending, as (expert, first row) pairs
-  int32_t* tiles = nullptr;
+  // at most tile_bm rows (tile_height) over each expert's segment, experts ascending, as {expert, first
+  // position, rows, 0}: all a block needs to know of its tile in one load
+  int4* tiles = nullptr;
   int32_t* n_tiles = nullptr;
   int tile_bm = 0;
 };
@@ -204,7 +217,7 @@ bool down1_fits(int type, int d, int K, int k, int s_K);
 int launch_down1(const Down1Args& a, hipStream_t st);
 
 
-// Grouped MFMA GEMM (prefill). Tiles come from `tiles` (pairs expert, first token; *n_tiles valid)
+// Grouped MFMA GEMM (prefill). Tiles come from `tiles` (DispatchScratch::tiles; *n_tiles valid)
 // over expert segments of the dispatch order, or, when tiles is null, cover T rows of one matrix.
 struct GemmArgs {
   const _Float16* A;       // activation rows, fp16 [*][K]
@@ -216,9 +229,8 @@ struct GemmArgs {
   int64_t row_bytes;       // bytes of one weight row of K elements
   int type;
   int N, K;
-  const int32_t* tiles;
+  const int4* tiles;
   const int32_t* n_tiles;
-  const int32_t* offsets;
   _Float16* out_h;         // gated: silu(gate) * up as fp16 [pos][N]
   float* out_y;            // plain: f32 [pos][N]
   int ksplit;              // plain projections: K split over this many blocks, partial sums to
@@ -262,9 +274,8 @@ struct GemmF32Args {
   const float* W0;         // gate (or the only) stack [E][N][K]
   const float* W1;         // up stack (gated) or null
   int N, K;
-  const int32_t* tiles;
+  const int4* tiles;
   const int32_t* n_tiles;
-  const int32_t* offsets;
   float* out;              // gated: h [pos][N]; plain: y [pos][N], part s at + s * part_stride
   int ksplit;              // plain projections: K split over this many blocks (1 when gated)
   int64_t part_stride;
