@@ -296,7 +296,7 @@ Layout layout(const ember_moe_layer* w, int T) {
                                                    (int)slots, w->d_ff, w->d)
                                  : 0;
   l.tailpart = o; o = align_up(o + (size_t)l.tail_parts * slots * 2 * w->d_ff * 4);
-  l.n_tiles = o; o = align_up(o + 4);
+  l.n_tiles = o; o = align_up(o + 64 + 9 * 4);  // the count; the XCDs' runs at + 64
   // the one-token slice launch's partial outputs [k][d_ff / 64][d]
   l.part = o; o = align_up(o + (slices_possible(w, T, l.mode, true) ? (size_t)w->k * (w->d_ff / 64) * w->d * 4 : 0));
   l.end = o;
@@ -470,6 +470,10 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     ds.tiles = at<int4>(scratch, l.tiles);
     ds.n_tiles = at<int32_t>(scratch, l.n_tiles);
     ds.tile_bm = gemm_tile_rows(l.mode == kSkinny);
+    if (l.mode == kGemm && T > ds.tile_bm) {  // (fewer tokens: one tile per expert, all alike)
+      ds.xcd = at<int32_t>(scratch, l.n_tiles + 64);
+      ds.xcd_tiles = (gemm_max_tiles(T, w->k, w->E) + 7) / 8;
+    }
   }
   float* h = at<float>(scratch, l.h);
   float* y = at<float>(scratch, l.y);
@@ -698,6 +702,7 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     g.K = d;
     g.tiles = tiles;
     g.n_tiles = n_tiles;
+    g.xcd = ds.xcd;
     g.out_h = h16;
     // the prefill pack serves the DMA tile kernels (256- and 64-token tiles alike)
     const PackLayout pl = pack_layout(d, d_ff, E, w->gate_type);

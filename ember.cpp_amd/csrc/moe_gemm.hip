@@ -269,16 +269,27 @@ __device__ inline int launch_mtiles(const GemmArgs& g, int bm) {
 }
 
 // XCD-balanced work item of block b for the 256-token-tile kernels: the W = M x NT x KS work items (m-tile
-// major, then n-tile, then K part) are cut into 8 equal runs, one per XCD (the hardware hands block b to
-// XCD b % 8), and XCD x's j-th block takes item x ceil(W / 8) + j. Every XCD gets the same share whatever
-// the (data-dependent) m-tile count, and the blocks an XCD holds at once mostly share one m-tile of
-// activations in its L2. False: no item (the grid is sized for the largest M).
-__device__ inline bool xcd_item(int M, int NT, int KS, int& mt, int& rem) {
-  const int W = M * NT * KS, C = (W + 7) / 8;
-  const int j = blockIdx.x / 8, w = (blockIdx.x % 8) * C + j;
-  if (j >= C || w >= W) return false;
-  mt = w / (NT * KS);
-  rem = w % (NT * KS);
+// major, then n-tile, then K part) are cut into 8 runs, one per XCD (the hardware hands block b to XCD b % 8), and
+// XCD x's j-th block takes item j of run x. The blocks an XCD holds at once mostly share one m-tile of
+// activations in its L2. The runs are of equal time where the dispatch estimated it (GemmArgs::xcd), else of
+// equal length: of Mixtral's ~20 m-tiles at T = 2048 four hold a few rows each, and runs of equal length left
+// some XCDs 280 full tiles and others 224 (CUs without a block a quarter of the time). False: no item (the
+// grid is sized for the largest M).
+__device__ inline bool xcd_item(const GemmArgs& g, int M, int NT, int KS, int& mt, int& rem) {
+  const int x = blockIdx.x % 8, j = blockIdx.x / 8, per = NT * KS;
+  int w, end;
+  if (g.xcd) {
+    const int p0 = g.xcd[x], p1 = g.xcd[x + 1];
+    w = (int)((int64_t)p0 * per / kXcdUnit) + j;
+    end = (int)((int64_t)p1 * per / kXcdUnit);
+  } else {
+    const int C = (M * per + 7) / 8;
+    w = x * C + j;
+    end = min(M * per, (x + 1) * C);
+  }
+  if (w >= end) return false;
+  mt = w / per;
+  rem = w % per;
   return true;
 }
 
@@ -347,7 +358,7 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
 
   // ---- the tile
   int mt, nt;
-  if (!xcd_item(launch_mtiles(g, GBM), NT, 1, mt, nt)) return;
+  if (!xcd_item(g, launch_mtiles(g, GBM), NT, 1, mt, nt)) return;
   int e, p0, rows;
   row_tile(g, mt, GBM, e, p0, rows);
   if (rows <= 0) return;
@@ -639,7 +650,7 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_q8_kernel(GemmArgs g, in
   } else {
     KS = GATED ? 1 : g.ksplit;
     int rem;
-    if (!xcd_item(launch_mtiles(g, GBM), NT, KS, mt, rem)) return;
+    if (!xcd_item(g, launch_mtiles(g, GBM), NT, KS, mt, rem)) return;
     nt = rem / KS;
     ks = rem % KS;
   }
@@ -1419,7 +1430,9 @@ int launch_gemm_fmt(const GemmArgs& g, int max_mtiles, hipStream_t st) {
     return EMBER_OK;
   }
   if (g.split_bf16) return EMBER_ERR_TYPE;  // the split path runs in the 64-token-tile kernel only
-  gemm_kernel<FMT, GATED><<<blocks, kGemmThreads, kGemmLds, st>>>(g, NT);
+  GemmArgs gk = g;
+  gk.xcd = nullptr;  // (this kernel's tiles take the same time whatever their rows)
+  gemm_kernel<FMT, GATED><<<blocks, kGemmThreads, kGemmLds, st>>>(gk, NT);
   return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
 }
 

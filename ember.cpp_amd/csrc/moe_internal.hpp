@@ -67,7 +67,12 @@ struct DispatchScratch {
   int4* tiles = nullptr;
   int32_t* n_tiles = nullptr;
   int tile_bm = 0;
+  // optional (null: none), with the tiles: the m-tile position, in kXcdUnit-ths of a tile, at which each XCD's run
+  // of the work begins, [9], runs of equal estimated time and at most xcd_tiles m-tiles
+  int32_t* xcd = nullptr;
+  int xcd_tiles = 0;
 };
+constexpr int kXcdUnit = 4096;
 
 int launch_router_logits(const float* x, int T, int d, int E, const float* R, float* logits, hipStream_t st);
 // Router logits of a small batch, one block per (expert, token) pair (router_block_logit's exact chains):
@@ -231,6 +236,7 @@ struct GemmArgs {
   int N, K;
   const int4* tiles;
   const int32_t* n_tiles;
+  const int32_t* xcd;      // DispatchScratch::xcd, or null
   _Float16* out_h;         // gated: silu(gate) * up as fp16 [pos][N]
   float* out_y;            // plain: f32 [pos][N]
   int ksplit;              // plain projections: K split over this many blocks, partial sums to

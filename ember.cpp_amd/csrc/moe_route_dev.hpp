@@ -554,6 +554,37 @@ __device__ inline void write_tiles(int q, int E, int cnt, int off, const Dispatc
   const int base = block_exclusive_scan(nt, tmp, &all);
   for (int i = 0; i < nt; ++i) ds.tiles[base + i] = make_int4(q, off + i * h, min(h, cnt - i * h), 0);
   if (q == 0) *ds.n_tiles = all;
+  if (!ds.xcd) return;
+  // Where the tiles' work reaches each eighth (DispatchScratch::xcd). The rest of a segment past whole tiles
+  // (at most 32 rows, tile_height) counts 6/13 of a tile, its measured time in the 256-token DMA kernels, when
+  // such rests are at least a sixth of the tiles (Mixtral-shaped T = 1050, most experts just past 256 rows, 1085 ->
+  // 955 us; T = 2048 1775 -> 1737). Otherwise all tiles count alike: runs of equal length that fill whole
+  // rounds of blocks are worth more (T = 1200, one rest in 16 tiles, 1132 us, weighted 1192; T = 512, weighted by
+  // 32-row steps, 512 -> 589).
+  const int rest = cnt - (nt - 1) * h;
+  const bool light = nt > 1 && rest <= 32;
+  const bool weigh = 6 * __syncthreads_count(light) >= all;
+  const int wh = 13 * 64, wl = light && weigh ? 6 * 64 : wh;
+  const int we = nt > 0 ? (nt - 1) * wh + wl : 0;
+  int wall = 0;
+  const int wbase = block_exclusive_scan(we, tmp, &wall);
+  for (int x = 1; x < 8; ++x) {
+    const int r = (int)((int64_t)wall * x / 8) - wbase;
+    if (r < 0 || r >= we) continue;  // one thread holds each eighth (none without tiles)
+    const int i = min(r / wh, nt - 1), wt = i < nt - 1 ? wh : wl;
+    tmp[x] = (base + i) * kXcdUnit + min((r - i * wh) * kXcdUnit / wt, kXcdUnit);
+  }
+  __syncthreads();
+  if (q == 0) {
+    int p = 0;
+    ds.xcd[0] = 0;
+    for (int x = 1; x < 8; ++x) {
+      const int cap = ds.xcd_tiles * kXcdUnit;
+      p = min(max(all ? tmp[x] : 0, max(p, all * kXcdUnit - (8 - x) * cap)), p + cap);
+      ds.xcd[x] = p;
+    }
+    ds.xcd[8] = all * kXcdUnit;
+  }
 }
 
 }  // namespace ember_moe
