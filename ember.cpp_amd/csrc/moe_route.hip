@@ -535,7 +535,7 @@ __global__ void __launch_bounds__(512) route_dispatch_small(const float* __restr
 // increasing q and the eight chains of a pair sit in eight consecutive lanes, combined by shuffles
 // in the reference's order. The eight pair groups of a wave read eight consecutive R rows per step,
 // padded to start 8 banks apart. Each thread converts PT + PE staged floats to double per PT * PE
-// FMAs, so the large-T variant takes 4 x 4 pairs.
+// FMAs.
 template <int GT, int GE, int PT, int PE, int KT>
 __global__ void __launch_bounds__(256) router_logits_chains(const float* __restrict__ x, const float* __restrict__ R,
                                                             float* __restrict__ logits, int T, int d, int E) {
@@ -641,6 +641,87 @@ __global__ void __launch_bounds__(256) router_logits_chains(const float* __restr
     }
 }
 
+// Router logits on the FP64 matrix cores: v_mfma_f64_16x16x4_f64 adds its four products to C one after another, k
+// = 0 .. 3, each rounded as an FMA (checked bitwise against the scalar chain), so with k running over four
+// consecutive q of one chain c (elements 8q + c) it continues that chain exactly as the reference does, for
+// 16 tokens x 16 experts at once. A wave runs four of the eight chains (a lane's four consecutive floats per q) of
+// NT such tiles side by side in the experts, a pair of waves shares them and their sums meet in LDS. Operands come
+// straight from memory, U steps of 32 elements ahead (the 16 rows of a wave's load are half lines, the pair's other
+// wave takes the other halves). Bound: the FP64 matrix rate, 48 TFLOP/s as measured (105 cycles per MFMA): E = 128,
+// d = 2048, T = 4096 takes 53 us of which 45 at that rate; the FMAs of router_logits_chains, which read both
+// operands from LDS for every few of them, took 88.
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+template <int NT, int U>
+__global__ void __launch_bounds__(256) router_logits_mfma(const float* __restrict__ x, const float* __restrict__ R,
+                                                          float* __restrict__ logits, int T, int d, int E) {
+  typedef float floatx4 __attribute__((ext_vector_type(4)));
+  __shared__ double part[4][NT][4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int tile = wave >> 1, share = wave & 1;  // two tiles per block, chains 4 share .. + 3
+  const int li = lane & 15, lk = lane >> 4;
+  const int t0 = blockIdx.x * 16, e0 = (blockIdx.y * 2 + tile) * 16 * NT;
+  const int nq = d / 8, steps = (nq + 3) / 4;
+  // (rows past the end repeat the last one, their logits are not stored)
+  const float* xp = x + (size_t)min(t0 + li, T - 1) * d + 4 * share;
+  const float* rp[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) rp[n] = R + (size_t)min(e0 + 16 * n + li, E - 1) * d + 4 * share;
+  doublex4 acc[NT][4];
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[n][c] = doublex4{0.0, 0.0, 0.0, 0.0};
+  struct Batch {
+    floatx4 a[U], b[U][NT];
+  };
+  // steps s0 .. s0 + U - 1; q past the end count as products 0 * 0, which leave a sum (never -0) as it is
+  auto load = [&](int s0, Batch& f) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const size_t o = 8 * (size_t)min(4 * (s0 + u) + lk, nq - 1);
+      f.a[u] = *reinterpret_cast<const floatx4*>(xp + o);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) f.b[u][n] = *reinterpret_cast<const floatx4*>(rp[n] + o);
+    }
+  };
+  auto run = [&](int s0, const Batch& f) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = 4 * (s0 + u) + lk < nq;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const double a = (double)(in ? f.a[u][c] : 0.0f);
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          acc[n][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)(in ? f.b[u][n][c] : 0.0f), acc[n][c], 0, 0, 0);
+      }
+    }
+  };
+  Batch f0, f1;
+  load(0, f0);
+  for (int s = 0; s < steps; s += 2 * U) {
+    load(s + U, f1);
+    run(s, f0);
+    load(s + 2 * U, f0);
+    run(s + U, f1);
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      part[wave][n][r][lane] = (acc[n][0][r] + acc[n][1][r]) + (acc[n][2][r] + acc[n][3][r]);
+  __syncthreads();
+  for (int i = share; i < NT * 4; i += 2) {  // the pair's waves finish every other row of their tiles
+    const int n = i / 4, r = i % 4;
+    const int t = t0 + 4 * r + lk, e = e0 + 16 * n + li;
+    if (t >= T || e >= E) continue;
+    const double sum = part[2 * tile][n][r][lane] + part[2 * tile + 1][n][r][lane];
+    double tail = 0.0;
+    for (int q = 8 * nq; q < d; ++q) tail = __builtin_fma((double)R[(size_t)e * d + q], (double)x[(size_t)t * d + q], tail);
+    logits[(size_t)t * E + e] = (float)(sum + tail);
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // Host-side launchers.
 
@@ -650,14 +731,19 @@ int launch_router_logits(const float* x, int T, int d, int E, const float* R, fl
   const int EG = max(1, min(router_lds_rows(d), (int)(((int64_t)T * E + 255) / 256)));
   const int64_t lds_blocks = (int64_t)T * ((E + EG - 1) / EG);
   if (d % 4 == 0 && ((E >= 16 && T >= 4) || (E >= 8 && T >= 64))) {
-    // one lane per chain; the largest tile that still gives >= 256 blocks: 16 x 32 pairs (E >= 32), 8 x 16
-    // (E >= 16), else 4 x 8 (with 8 to 15 experts the staged-row kernels below stay ahead up to a few
-    // dozen tokens). Measured router times, 4 x 8 / 8 x 16 / 16 x 32: C3-shaped (E = 128, d = 2048) T = 128
-    // 14.4 / 17.6 / 34.0 us, T = 256 21.1 / 18.9, T = 512 34.8 / 25.7 / 34.4, T = 1024 - / 40.6 / 36.5;
-    // C4-shaped (E = 64) T = 256 13.5 / 16.9, T = 512 20.4 / 18.0, T = 1024 32.4 / 24.7
-    const int64_t b16 = (int64_t)((T + 15) / 16) * ((E + 31) / 32), b8 = (int64_t)((T + 7) / 8) * ((E + 15) / 16);
-    if (E >= 32 && b16 >= 256) {
-      router_logits_chains<4, 8, 4, 4, 128><<<dim3((T + 15) / 16, (E + 31) / 32), 256, 0, st>>>(x, R, logits, T, d, E);
+    // The FP64 matrix cores from 64 Ki pairs on, where their waves (two per 16 x 16 pairs, or per 16 x 32 past
+    // 128 Ki pairs: one round on the chip's 1024 SIMDs) take no longer than the FMAs' blocks. FMA / MFMA, same bits: E =
+    // 128, d = 2048 T = 512 20.9 / 18.0 us, T = 1024 31.0 / 18.4, T = 2048 45.9 / 31.9, T = 4096 87.8 / 52.6; E = 64
+    // T = 1024 19.9 / 17.9, T = 1500 25.1 / 18.1; below, E = 64 T = 512 14.0 / 17.8; E = 8, half of whose 16 columns
+    // would idle, d = 4096 T = 2048 17.3 / 31.7.
+    // Else one lane per chain; the largest tile that still gives >= 256 blocks: 8 x 16 (E >= 16), else 4 x 8
+    // (with 8 to 15 experts the staged-row kernels below stay ahead up to a few dozen tokens). 4 x 8 / 8 x 16: E = 128,
+    // d = 2048 T = 128 14.4 / 17.6 us, T = 256 21.1 / 18.9; E = 64 T = 256 13.5 / 16.9, T = 512 20.4 / 18.0
+    const int64_t b8 = (int64_t)((T + 7) / 8) * ((E + 15) / 16), pairs = (int64_t)T * E;
+    if (E >= 32 && d >= 64 && pairs > 131072) {
+      router_logits_mfma<2, 2><<<dim3((T + 15) / 16, (E + 63) / 64), 256, 0, st>>>(x, R, logits, T, d, E);
+    } else if (E >= 32 && d >= 64 && pairs >= 65536) {
+      router_logits_mfma<1, 4><<<dim3((T + 15) / 16, (E + 31) / 32), 256, 0, st>>>(x, R, logits, T, d, E);
     } else if (E >= 16 && b8 >= 256) {
       router_logits_chains<4, 8, 2, 2, 256><<<dim3((T + 7) / 8, (E + 15) / 16), 256, 0, st>>>(x, R, logits, T, d, E);
     } else {
