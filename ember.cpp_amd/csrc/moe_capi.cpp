@@ -85,13 +85,18 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
   } else if (avg_m <= 2.0) {
     return kGemv;
   }
-  // (one dense matrix, the shared expert: the 64-token tiles, split over K, up to 1024 rows; C4 shape
-  // T = 512: 139 vs 201 us on the 256-token tiles, T = 2048: 234 vs 208)
-  // packed BF16 routed experts: the 256-token tiles from ~32 tokens per expert (C4-shaped, 64-token /
-  // 256-token tiles: T = 256 (24 per expert) 184 / 213 us, T = 512 (48) 270 / 228, T = 1024 426 / 392,
-  // T = 2048 716 / 553)
-  const bool bf16_packed = packed && type_in == EMBER_TYPE_BF16 && type_out == EMBER_TYPE_BF16 && E > 1;
-  if (avg_m <= (E == 1 ? 1024.0 : bf16_packed ? 32.0 : 96.0)) return kSkinny;
+  // (one dense matrix, the shared expert: the 64-token tiles, split over K, up to 800 rows; DeepSeek-shaped layer,
+  // 64- / 256-token tiles: BF16 T = 700 270 / 293 us, T = 850 353 / 302; F16 T = 850 376 / 379, T = 1000 406 / 403)
+  // BF16 (packed) and F16 routed experts: the 64-token tiles stream the weights best while most experts fit one,
+  // up to 60 rows per expert (Mixtral-shaped BF16 T = 160 (40) 589 / 733, T = 256 (64) 789 / 784, T = 384 976 / 848)
+  // and, with 32 experts and more, whose counts spread further, up to 28 (DeepSeek-shaped BF16 T = 256 (24) 182 /
+  // 196, T = 300 (28) 213 / 183; F16 T = 256 188 / 190, T = 300 215 / 180; Qwen-shaped T = 512 (32) 350 / 346, T = 1500 528
+  // / 456); up to 250 where the 256-token gate/up launch would not give every CU a block (d_ff 2816, E 8, F16: T = 400
+  // (100) 99 / 126, T = 768 (192) 134 / 153, T = 1500 (375) 212 / 180)
+  const double most64 = E * ((K_out + 127) / 128) < 256 ? 250.0 : E >= 32 ? 28.0 : 60.0;
+  if (half && (packed || type_in == EMBER_TYPE_F16 || type_out == EMBER_TYPE_F16) && E > 1)
+    return avg_m <= most64 ? kSkinny : kGemm;
+  if (avg_m <= (E > 1 ? 96.0 : half ? 800.0 : 1024.0)) return kSkinny;
   if (type_in == EMBER_TYPE_BF16 && type_out == EMBER_TYPE_BF16 && !packed) return kSkinny;
   return kGemm;
 }

@@ -14,8 +14,8 @@
 //
 // Kernels: gemm_dma_q8_kernel (Q8_0 rows or the prefill pack's Q8_0 / Q4_K tiles; 256-token tiles,
 // weights and activations loaded straight into LDS), gemm_dma64_q8_kernel (the same formats, 64-token
-// tiles), gemm_kernel and gemm_skinny_kernel (register-staged 256- / 64-token tiles for the other
-// formats). Tiles are (expert, first token) pairs from a table the dispatch step writes (dense rows:
+// tiles), gemm_dma_half_kernel (BF16 and F16 rows, 256-token tiles), gemm_kernel and gemm_skinny_kernel
+// (register-staged 256- / 64-token tiles for the other formats). Tiles are (expert, first token) pairs from a table the dispatch step writes (dense rows:
 // consecutive token ranges); grids are sized for the most tiles a call can have, blocks take their work
 // items XCD-balanced from the device-side tile count, and blocks without one exit at once. The down
 // projection can split K over blocks (partial sums added in order by the combine); the 256-token gate/up
@@ -375,13 +375,11 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
     a_src = g.A + (size_t)(g.perm ? g.perm[p] / g.k : p) * K + 32 * lh;
   }
   const uint8_t* b_row = nullptr;
-  float b_sc = 1.0f;  // BF16: 2^-(the row's exponent)
   {
     const int b_g = GATED ? (lr >> 7) : 0;
     const int b_n = n0 + (GATED ? (lr & 127) : lr);
     if (b_n < N) {
       b_row = static_cast<const uint8_t*>(b_g ? g.W1 : g.W0) + (int64_t)e * g.expert_stride + (int64_t)b_n * g.row_bytes;
-      if (FMT == EMBER_TYPE_BF16) b_sc = __builtin_ldexpf(1.0f, -w_exp_of(b_g ? g.w_exp1 : g.w_exp0, e, N, b_n));
     }
   }
 
@@ -405,10 +403,7 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
     for (int v = 0; v < 4; ++v) *reinterpret_cast<u32x4*>(&As[lr * LDK + 32 * lh + 8 * v]) = a_reg[v];
     uint32_t dq[16];
     if (b_row) {
-      if constexpr (FMT == EMBER_TYPE_BF16)
-        bf16_to_f16_scaled(b_raw, b_sc, dq);
-      else
-        D::decode_half(b_raw, kt, lh, dq);
+      D::decode_half(b_raw, kt, lh, dq);
     } else {
 #pragma unroll
       for (int w = 0; w < 16; ++w) dq[w] = 0u;
@@ -429,6 +424,7 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
         for (int r = 0; r < 16; ++r) acc[q][i][jn][r] = 0.0f;
 
   auto mfma_stage = [&](int stage) {
+    if (64 * wm >= rows) return;  // (wave-uniform) this wave's rows hold no tokens
     const _Float16* As = smem + stage * kStageHalves;
     const _Float16* Bs = As + GBM * LDK;
 #pragma unroll
@@ -469,9 +465,6 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
     for (int jn = 0; jn < WN; ++jn) {
       const int n = n0 + wn * (WN * 32) + 32 * jn + (lane & 31);
       if (n >= N) continue;
-      const int we0 = FMT == EMBER_TYPE_BF16 ? w_exp_of(g.w_exp0, e, N, n) : 0;
-      const int we1 = FMT == EMBER_TYPE_BF16 && GATED ? w_exp_of(g.w_exp1, e, N, n) : 0;
-      const int weh = FMT == EMBER_TYPE_BF16 && GATED && g.w_hexp ? (int)g.w_hexp[e] : 0;
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii)
 #pragma unroll
@@ -481,10 +474,9 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
           const size_t o = (size_t)(p0 + m) * N + n;
           const int ex = s_rexp[m];
           if constexpr (GATED) {
-            store_h(g, o, p0 + m, ex, __builtin_ldexpf(acc[0][i][jn][4 * ii + jj], we0),
-                    __builtin_ldexpf(acc[1][i][jn][4 * ii + jj], we1), n == n0, weh);
+            store_h(g, o, p0 + m, ex, acc[0][i][jn][4 * ii + jj], acc[1][i][jn][4 * ii + jj], n == n0);
           } else {
-            g.out_y[o] = unscale_y(__builtin_ldexpf(acc[0][i][jn][4 * ii + jj], we0), ex);
+            g.out_y[o] = unscale_y(acc[0][i][jn][4 * ii + jj], ex);
           }
         }
     }
@@ -888,6 +880,208 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_q8_kernel(GemmArgs g, in
             }
           } else {
             g.out_y[ks * g.part_stride + o] = unscale_y(acc[i][jn][4 * ii + jj], ex);
+          }
+        }
+    }
+}
+
+// The 256-token DMA kernel for BF16 (with the row exponents of a prefill pack) and F16 rows: gemm_dma_q8_kernel's
+// layout (2 (M) x 4 (N) waves of 128 x 64, subtiles past the tile's rows skipped, XCD runs, K split of the plain
+// projection) with K tiles of 32 columns, so that both operands of a stage (16 KiB each) fit a ring of four,
+// three tiles in flight. A tile row is 64 bytes, four granules, XOR-swizzled so that the 16 rows one read pass
+// touches fall on distinct banks. A B fragment is one 16-byte read; BF16 values are scaled by the row's power of two
+// and rounded to fp16 on the way to the MFMA, as the register-staged kernel does, whose outputs these equal
+// bit for bit. That kernel multiplied 256 rows whatever a tile held and drained its loads every K tile:
+// DeepSeek-shaped BF16 T = 1500 (140 rows per expert) 524 -> 429 us, F16 474 -> 375, Mixtral-shaped BF16 T = 256 996
+// -> 776, Qwen-shaped BF16 T = 4000 864 -> 720.
+constexpr int kHalfBK = 32, kHalfStages = 4;
+constexpr int kHalfA = GBM * kHalfBK * 2, kHalfStage = 2 * kHalfA;  // 256 activation rows, 256 weight rows
+constexpr size_t kHalfLds = (size_t)kHalfStages * kHalfStage;
+constexpr int kHalfInst = kHalfA / 1024 / 8;  // 1 KiB loads per wave and operand
+
+template <int FMT, bool GATED>
+__global__ void __launch_bounds__(kDmaThreads) gemm_dma_half_kernel(GemmArgs g, int NT) {
+  constexpr int BN = GATED ? 128 : 256, NS = kHalfStages;
+  extern __shared__ __align__(16) uint8_t dsm[];
+  const int KS = GATED ? 1 : g.ksplit;
+  int mt, rem, e, p0, rows;
+  if (!xcd_item(g, launch_mtiles(g, GBM), NT, KS, mt, rem)) return;
+  const int nt = rem / KS, ks = rem % KS;
+  row_tile(g, mt, GBM, e, p0, rows);
+  if (rows <= 0) return;
+  const int n0 = nt * BN, K = g.K, N = g.N;
+  const int nk_all = K / kHalfBK;
+  const int kt0 = ks * nk_all / KS, nk = (ks + 1) * nk_all / KS - kt0;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 2, wn = wave & 3;
+  const int msub = min(4, max(0, (rows - 128 * wm + 31) >> 5));
+
+  // DMA sources: load i of a wave fills granules 64 (2 w + i) + lane of either operand; granule gi is row gi / 4,
+  // slot gi % 4, holding K granule slot ^ ((row / 4) % 4). Rows past the tile (the matrix) repeat its last row.
+  const uint8_t* srcA[kHalfInst];
+  const uint8_t* srcB[kHalfInst];
+#pragma unroll
+  for (int i = 0; i < kHalfInst; ++i) {
+    const int gi = 64 * (kHalfInst * wave + i) + lane, r = gi >> 2, kg = (gi & 3) ^ ((r >> 2) & 3);
+    const int p = p0 + min(r, rows - 1);
+    srcA[i] = reinterpret_cast<const uint8_t*>(g.A + (size_t)(g.perm ? g.perm[p] / g.k : p) * K + 8 * kg);
+    const int q = GATED ? (r >> 7) : 0, n = min(n0 + (GATED ? (r & 127) : r), N - 1);
+    srcB[i] = static_cast<const uint8_t*>(q ? g.W1 : g.W0) + (int64_t)e * g.expert_stride + (int64_t)n * g.row_bytes + 16 * kg;
+  }
+  // tile kt (clamped: tiles past the end reload the last, never multiplied) into the stage at byte `st`.
+  // NOA: this wave's activation rows (32 w .. 32 w + 31) lie past the tile's tokens, so it loads none.
+  auto issue = [&](int kt, int st, auto NOAc) {
+    const size_t o = (size_t)(kt0 + min(kt, nk - 1)) * kHalfBK * 2;
+#pragma unroll
+    for (int i = 0; i < kHalfInst; ++i) {
+      if constexpr (!decltype(NOAc)::value) lds_dma16(srcA[i] + o, dsm + st + 1024 * (kHalfInst * wave + i));
+      lds_dma16(srcB[i] + o, dsm + st + kHalfA + 1024 * (kHalfInst * wave + i));
+    }
+  };
+
+  floatx16 acc[4][2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int jn = 0; jn < 2; ++jn)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][jn][r] = 0.0f;
+
+  const int h = lane >> 5, li = lane & 31;
+  // this lane's LDS bytes within a stage: its activation row of subtile 0 at K step ks (subtile i 2 KiB on) and
+  // its weight row of subtile jn; rows a multiple of 16 apart share the swizzle
+  uint32_t offA[2], offB[2];
+  float sc[2];  // BF16: 2^-(the weight row's exponent)
+#pragma unroll
+  for (int s = 0; s < 2; ++s) offA[s] = 64 * (wm * 128 + li) + 16 * ((2 * s + h) ^ ((li >> 2) & 3));
+#pragma unroll
+  for (int jn = 0; jn < 2; ++jn) {
+    const int br = GATED ? jn * 128 + wn * 32 + li : wn * 64 + 32 * jn + li;
+    offB[jn] = kHalfA + 64 * br - 64 * (wm * 128 + li);  // (plus offA)
+    const int n = n0 + (GATED ? wn * 32 + li : br);
+    sc[jn] = FMT == EMBER_TYPE_BF16 ? __builtin_ldexpf(1.0f, -w_exp_of(GATED && jn ? g.w_exp1 : g.w_exp0, e, N, min(n, N - 1)))
+                                    : 1.0f;
+  }
+  auto barrier = [] {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // The K loop, rotated as gemm_dma_q8_kernel's: the barrier (tile kt + 1 has landed, tile kt is read) sits
+  // between the two K steps of tile kt
+  auto k_loop = [&](auto MSc, auto NOAc) {
+    constexpr int MS = decltype(MSc)::value;
+    constexpr int kInst = (decltype(NOAc)::value ? 1 : 2) * kHalfInst;
+    half8 fa[2][MS > 0 ? MS : 1], fb[2][2];
+    u32x4 raw[2];
+    auto read = [&](int st, int s, half8 (&a)[MS > 0 ? MS : 1]) {
+#pragma unroll
+      for (int jn = 0; jn < 2; ++jn) raw[jn] = *reinterpret_cast<const u32x4*>(dsm + st + offA[s] + offB[jn]);
+#pragma unroll
+      for (int i = 0; i < MS; ++i) a[i] = *reinterpret_cast<const half8*>(dsm + st + offA[s] + 2048 * i);
+    };
+    auto decode = [&](half8 (&b)[2]) {
+#pragma unroll
+      for (int jn = 0; jn < 2; ++jn) {
+        if constexpr (FMT == EMBER_TYPE_BF16) {
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            b[jn][2 * w] = (_Float16)(as_f32(raw[jn][w] << 16) * sc[jn]);
+            b[jn][2 * w + 1] = (_Float16)(as_f32(raw[jn][w] & 0xffff0000u) * sc[jn]);
+          }
+        } else {
+          b[jn] = __builtin_bit_cast(half8, raw[jn]);
+        }
+      }
+    };
+    auto mfmas = [&](const half8 (&a)[MS > 0 ? MS : 1], const half8 (&b)[2]) {
+#pragma unroll
+      for (int i = 0; i < MS; ++i)
+#pragma unroll
+        for (int jn = 0; jn < 2; ++jn)
+          acc[i][jn] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[i], b[jn], acc[i][jn], 0, 0, 0);
+    };
+#pragma unroll
+    for (int t = 0; t < NS - 1; ++t) issue(t, t * kHalfStage, NOAc);
+    wait_vmcnt<(NS - 2) * kInst>();
+    barrier();
+    if constexpr (MS > 0) {
+      read(0, 0, fa[0]);
+      decode(fb[0]);
+    }
+    int cur = 0, fill = (NS - 1) * kHalfStage;
+    for (int kt = 0; kt < nk; ++kt) {
+      const int nxt = cur == (NS - 1) * kHalfStage ? 0 : cur + kHalfStage;
+      if constexpr (MS > 0) read(cur, 1, fa[1]);
+      issue(kt + NS - 1, fill, NOAc);
+      if constexpr (MS > 0) {
+        mfmas(fa[0], fb[0]);
+        decode(fb[1]);
+      }
+      wait_vmcnt<(NS - 2) * kInst>();
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's reads of tile kt are complete
+      barrier();
+      if constexpr (MS > 0) {
+        read(nxt, 0, fa[0]);
+        mfmas(fa[1], fb[1]);
+        decode(fb[0]);
+      }
+      fill = cur;
+      cur = nxt;
+    }
+  };
+  __shared__ int s_rexp[GBM];
+  load_row_exps(g, p0, rows, s_rexp);
+  using A1 = std::integral_constant<bool, false>;
+  using A0 = std::integral_constant<bool, true>;
+  using M4 = std::integral_constant<int, 4>;
+  using M3 = std::integral_constant<int, 3>;
+  using M2 = std::integral_constant<int, 2>;
+  using M1 = std::integral_constant<int, 1>;
+  using M0 = std::integral_constant<int, 0>;
+  if (32 * wave >= rows) {  // (four subtiles of a half fill all of its waves' activation rows)
+    switch (msub) {
+      case 3: k_loop(M3{}, A0{}); break;
+      case 2: k_loop(M2{}, A0{}); break;
+      case 1: k_loop(M1{}, A0{}); break;
+      default: k_loop(M0{}, A0{}); break;
+    }
+  } else {
+    switch (msub) {
+      case 4: k_loop(M4{}, A1{}); break;
+      case 3: k_loop(M3{}, A1{}); break;
+      case 2: k_loop(M2{}, A1{}); break;
+      case 1: k_loop(M1{}, A1{}); break;
+      default: k_loop(M0{}, A1{}); break;
+    }
+  }
+  wait_vmcnt<0>();  // no DMA may still target LDS when the block exits
+  __syncthreads();  // the row exponents are visible
+
+  // ---- epilogue: lane holds column (lane & 31) of each 32x32 subtile, rows 8*ii + 4*(lane>>5) + jj
+  const int weh = FMT == EMBER_TYPE_BF16 && GATED && g.w_hexp ? (int)g.w_hexp[e] : 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int jn = 0; jn < (GATED ? 1 : 2); ++jn) {
+      const int n = n0 + (GATED ? wn * 32 : wn * 64 + 32 * jn) + li;
+      if (n >= N) continue;
+      const int we0 = FMT == EMBER_TYPE_BF16 ? w_exp_of(g.w_exp0, e, N, n) : 0;
+      const int we1 = FMT == EMBER_TYPE_BF16 && GATED ? w_exp_of(g.w_exp1, e, N, n) : 0;
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const int m = wm * 128 + 32 * i + 8 * ii + 4 * h + jj;
+          if (m >= rows) continue;
+          const size_t o = (size_t)(p0 + m) * N + n;
+          const int ex = s_rexp[m];
+          if constexpr (GATED) {
+            store_h(g, o, p0 + m, ex, __builtin_ldexpf(acc[i][0][4 * ii + jj], we0),
+                    __builtin_ldexpf(acc[i][1][4 * ii + jj], we1), n == n0, weh);
+          } else {
+            g.out_y[ks * g.part_stride + o] = unscale_y(__builtin_ldexpf(acc[i][jn][4 * ii + jj], we0), ex);
           }
         }
     }
@@ -1393,16 +1587,21 @@ int launch_dma(int type, const GemmArgs& gk, int NT, unsigned nb, hipStream_t st
 template <int FMT, bool GATED>
 int launch_gemm_fmt(const GemmArgs& g, int max_mtiles, hipStream_t st) {
   constexpr int BN = GATED ? 128 : 256;
-  static const bool lds_ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<FMT, GATED>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
-  if (!lds_ok) return EMBER_ERR_LAUNCH;
   const int NT = (g.N + BN - 1) / BN;
   const int mgroups = (max_mtiles + 7) / 8;
   const unsigned blocks = (unsigned)(8 * mgroups * NT);
   if (max_mtiles == 0 || NT == 0) return EMBER_OK;
-  if (dma_path(FMT, g.Wp != nullptr)) {
-    GemmArgs gk = g;
+  GemmArgs gk = g;
+  if constexpr (FMT == EMBER_TYPE_BF16 || FMT == EMBER_TYPE_F16) {
+    if (g.split_bf16) return EMBER_ERR_TYPE;  // the split path runs in the 64-token-tile kernel only
+    static const bool ok =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_half_kernel<FMT, GATED>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kHalfLds) == hipSuccess;
+    if (!ok) return EMBER_ERR_LAUNCH;
+    if (GATED || gk.ksplit < 1) gk.ksplit = 1;
+    gemm_dma_half_kernel<FMT, GATED><<<blocks * (unsigned)gk.ksplit, kDmaThreads, kHalfLds, st>>>(gk, NT);
+    return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
+  } else if (dma_path(FMT, g.Wp != nullptr)) {
     if (GATED || gk.ksplit < 1) gk.ksplit = 1;
     const bool tail = GATED && gk.tail_parts > 1 && gk.slots > 0 && gk.part_h && gk.tiles;
     if (!tail) gk.tail_parts = 1;
@@ -1428,12 +1627,15 @@ int launch_gemm_fmt(const GemmArgs& g, int max_mtiles, hipStream_t st) {
       if (hipGetLastError() != hipSuccess) return EMBER_ERR_LAUNCH;
     }
     return EMBER_OK;
+  } else {
+    static const bool lds_ok =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<FMT, GATED>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
+    if (!lds_ok) return EMBER_ERR_LAUNCH;
+    gk.xcd = nullptr;  // (this kernel's tiles take about the same time whatever their rows)
+    gemm_kernel<FMT, GATED><<<blocks, kGemmThreads, kGemmLds, st>>>(gk, NT);
+    return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
   }
-  if (g.split_bf16) return EMBER_ERR_TYPE;  // the split path runs in the 64-token-tile kernel only
-  GemmArgs gk = g;
-  gk.xcd = nullptr;  // (this kernel's tiles take the same time whatever their rows)
-  gemm_kernel<FMT, GATED><<<blocks, kGemmThreads, kGemmLds, st>>>(gk, NT);
-  return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
 }
 
 template <bool GATED>

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T", [256, 257, 288, 289, 300, 513, 545, 700])
-@pytest.mark.parametrize("wtype,pack,E", [(em.Q8_0, True, 2), (em.Q8_0, False, 3), (em.Q4_K, True, 2), (em.BF16, True, 2)])
+@pytest.mark.parametrize("wtype,pack,E", [(em.Q8_0, True, 2), (em.Q8_0, False, 3), (em.Q4_K, True, 2), (em.BF16, True, 2), (em.F16, False, 2)])
 def test_tile_heights(gpu, monkeypatch, wtype, pack, E, T):
     spec = em.LayerSpec(d=256, d_ff=512, E=E, k=E, wtype=wtype, seed=5)
     hl = em.make_host_layer(spec)
@@ -27,6 +27,24 @@ def test_tile_heights(gpu, monkeypatch, wtype, pack, E, T):
         assert same_bits(y[a:a + 200], run_gpu(hl, x[a:a + 200], pack=pack)), a
     monkeypatch.setenv("EMBER_KSPLIT", "4")
     assert rel_l2(run_gpu(hl, x, pack=pack), y) < 1e-5
+
+
+@pytest.mark.parametrize("T", [31, 32, 33, 96, 97, 129, 256, 300])
+@pytest.mark.parametrize("wtype,pack,shared", [(em.BF16, True, 0), (em.F16, False, 0), (em.BF16, True, 192)])
+def test_half_tiles_ragged(gpu, monkeypatch, wtype, pack, shared, T):
+    """The BF16 / F16 256-token tiles: subtiles and activation loads past a tile's rows left out, weight rows past
+    d_ff and d (320 = 2.5 x 128, 192 < 256), an even and an odd number of 32-column K tiles per part, a dense shared
+    expert, against the oracle at the fp16 operands' 2e-3."""
+    spec = em.LayerSpec(d=192, d_ff=320, E=3, k=3, wtype=wtype, seed=T, d_ff_shared=shared)
+    hl = em.make_host_layer(spec)
+    x = em.make_input(spec, T)
+    monkeypatch.setenv("EMBER_MOE_PATH", "gemm")
+    monkeypatch.setenv("EMBER_MOE_SHARED_PATH", "gemm")
+    print(f"half tiles {em.TYPE_NAMES[wtype]} T={T} shared={shared}", flush=True)
+    y = run_gpu(hl, x, pack=pack)
+    assert np.isfinite(y).all()
+    assert rel_l2(y, run_oracle(hl, x)) < 2e-3
+    assert same_bits(y, run_gpu(hl, x, pack=pack))
 
 
 @pytest.mark.parametrize("T", [1050, 2048])
