@@ -219,6 +219,8 @@ struct Layout {
   size_t tailpart;                        // the 256-token gate/up launch's tail partials
   size_t rfast;                           // the proven-picks router's planes, row scales and bounds
   int tail_parts;                         // their parts (0: no tail split)
+  bool short_tiles;                       // the 256-token path's tiles hold at most 64 rows
+  int mtiles;                             // most row tiles of the routed launches
   int mode, mode_shared;                  // PathMode of the routed experts and of the shared expert
   int ks_sh_gu, ks_sh_dn;                 // K split of the shared expert's 64-token-tile launches
   RouteLayout r;
@@ -278,9 +280,10 @@ Layout layout(const ember_moe_layer* w, int T) {
   }
   l.ys = o; o = align_up(o + (w->d_ff_shared > 0 ? (size_t)l.ks_sh_dn * T * w->d * 4 : 0));
   l.shpart = o; o = align_up(o + (l.ks_sh_gu > 1 ? (size_t)l.ks_sh_gu * T * 2 * w->d_ff_shared * 4 : 0));
-  const size_t tiles = l.mode == kGemm     ? (size_t)gemm_max_tiles(T, w->k, w->E)
-                       : l.mode == kSkinny ? (size_t)gemm_skinny_max_tiles(T, w->k, w->E)
-                                           : 0;
+  l.short_tiles = l.mode == kGemm && gemm_short_tiles(w->gate_type, w->prefill_pack != nullptr, T, w->k, w->E, w->d_ff);
+  l.mtiles = l.mode == kGemv                      ? 0
+             : l.mode == kGemm && !l.short_tiles ? gemm_max_tiles(T, w->k, w->E)
+                                                 : gemm_skinny_max_tiles(T, w->k, w->E);
   // (the F32 tiles read x and write h in f32: none of the converted activations below)
   const bool mfma = l.mode != kGemv && !f32_stacks(w->gate_type, w->down_type);
   const bool mfma_sh = w->d_ff_shared > 0 && l.mode_shared != kGemv && !f32_sh;
@@ -295,7 +298,7 @@ Layout layout(const ember_moe_layer* w, int T) {
   l.hexp = o; o = align_up(o + (mfma && !sp ? slots * 4 : 0));
   l.hs16 = o; o = align_up(o + (mfma_sh ? (size_t)T * w->d_ff_shared * (sp_sh ? 4 : 2) : 0));
   l.hsexp = o; o = align_up(o + (mfma_sh && !sp_sh ? (size_t)T * 4 : 0));
-  l.tiles = o; o = align_up(o + tiles * 16);
+  l.tiles = o; o = align_up(o + (size_t)l.mtiles * 16);
   // the routed gate/up's tail split (256-token tiles): raw partial gate / up dots [parts][T k][2 d_ff]
   l.tail_parts = l.mode == kGemm ? gemm_tail_parts(w->gate_type, w->prefill_pack != nullptr && !pack_bf16,
                                                    (int)slots, w->d_ff, w->d)
@@ -474,10 +477,10 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
   if (l.mode != kGemv) {  // the dispatch also writes the MFMA GEMMs' tile table
     ds.tiles = at<int4>(scratch, l.tiles);
     ds.n_tiles = at<int32_t>(scratch, l.n_tiles);
-    ds.tile_bm = gemm_tile_rows(l.mode == kSkinny);
-    if (l.mode == kGemm && T > ds.tile_bm) {  // (fewer tokens: one tile per expert, all alike)
+    ds.tile_bm = gemm_tile_rows(l.mode == kSkinny || l.short_tiles);
+    if (l.mode == kGemm && !l.short_tiles && T > ds.tile_bm) {  // (fewer tokens: one tile per expert, all alike)
       ds.xcd = at<int32_t>(scratch, l.n_tiles + 64);
-      ds.xcd_tiles = (gemm_max_tiles(T, w->k, w->E) + 7) / 8;
+      ds.xcd_tiles = (l.mtiles + 7) / 8;
     }
   }
   float* h = at<float>(scratch, l.h);
@@ -665,7 +668,7 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     g.n_tiles = ds.n_tiles;
     g.out = h;
     g.ksplit = 1;
-    const int mt = gemm_skinny_max_tiles(T, k, E);
+    const int mt = l.mtiles;
     if ((s = launch_gemm_f32(g, true, mt, st))) return s;
     mark(ev, 4, st);
     g.A = h;
@@ -718,7 +721,8 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
       g.w_exp1 = wexp(bx.up);
       g.w_hexp = wexp(bx.hmax);
     }
-    const int mt = skinny ? gemm_skinny_max_tiles(T, k, E) : gemm_max_tiles(T, k, E);
+    const int mt = l.mtiles;
+    g.short_tiles = l.short_tiles;
     if (!skinny && l.tail_parts > 1) {  // the tail round's tiles split over K
       g.part_h = at<float>(scratch, l.tailpart);
       g.part_rows = T * k;

@@ -15,8 +15,8 @@
 // Kernels: gemm_dma_q8_kernel (Q8_0 rows or the prefill pack's Q8_0 / Q4_K tiles; 256-token tiles,
 // weights and activations loaded straight into LDS), gemm_dma64_q8_kernel (the same formats, 64-token
 // tiles), gemm_dma_half_kernel (BF16 and F16 rows, 256-token tiles), gemm_kernel and gemm_skinny_kernel
-// (register-staged 256- / 64-token tiles for the other formats). Tiles are (expert, first token) pairs from a table the dispatch step writes (dense rows:
-// consecutive token ranges); grids are sized for the most tiles a call can have, blocks take their work
+// (register-staged 256- / 64-token tiles for the other formats). Tiles are (expert, first token, rows) from a
+// table the dispatch step writes (dense rows: consecutive token ranges); grids are sized for the most tiles a call can have, blocks take their work
 // items XCD-balanced from the device-side tile count, and blocks without one exit at once. The down
 // projection can split K over blocks (partial sums added in order by the combine); the 256-token gate/up
 // launch splits only the tiles of its partial last round (the tail split), which a fixup launch finishes.
@@ -485,8 +485,8 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
 // ---------------------------------------------------------------------------------------------
 // Q8_0 grouped GEMM with direct global->LDS tile loads. Tiles of 256 tokens x 256 weight rows x 64 K
 // run through a ring of three LDS stages that global_load_lds fills without passing through
-// registers, so two tiles are in flight while one is multiplied (launches of at most 64 tokens: 64-row
-// activation stages and five stages, four tiles in flight). Every wave loads a share of both
+// registers, so two tiles are in flight while one is multiplied (tiles of at most 64 rows: 64-row
+// activation stages, DmaRing). Every wave loads a share of both
 // operands: the activation tile as 16-byte granules XOR-swizzled by row pair (the 16 rows that one
 // 16-lane pass of ds_read_b128 reads fall on distinct bank groups of the 64-bank LDS), the weight
 // tile in its Q8_0 bytes: the 68 bytes of a row's K tile as five 16-byte granules, the fifth
@@ -495,17 +495,13 @@ __global__ void __launch_bounds__(kGemmThreads) gemm_kernel(GemmArgs g, int NT) 
 // 32 up columns, so SwiGLU pairs meet in one wave) and decodes its own B fragments from the Q8_0
 // bytes straight into MFMA operands (fp16 d * q, one rounding, as the decoders above).
 typedef __attribute__((address_space(3))) void lds_void_t;
-constexpr int kDmaThreads = 512, kDmaStages = 3;
-constexpr int kDmaRowB = 80;                     // LDS bytes of one weight row's K tile
+constexpr int kDmaThreads = 512;
+constexpr int kDmaRowB = 80;                     // LDS bytes of one ggml row's K tile
 constexpr int kDmaA = GBM * GBK * 2;             // activation bytes per stage (32 KiB)
-constexpr int kDmaB = 256 * kDmaRowB;            // weight bytes per stage (20 KiB)
-constexpr int kDmaStage = kDmaA + kDmaB;
-constexpr size_t kDmaLds = (size_t)kDmaStages * kDmaStage;
-// launches of at most 64 tokens (every segment, hence every tile, holds at most 64 rows: a token picks an
-// expert once): 64 activation rows per stage (8 KiB) and five stages, four tiles in flight
-constexpr int kDmaStagesShort = 5, kShortRows = 64;
+constexpr int kDmaB = 256 * kDmaRowB;            // weight bytes per stage (20 KiB; the packs' tiles are smaller)
+// short tiles, of at most 64 rows: 64 activation rows per stage (8 KiB)
+constexpr int kShortRows = 64;
 constexpr int kDmaAShort = kShortRows * GBK * 2;
-constexpr size_t kDmaLdsShort = (size_t)kDmaStagesShort * (kDmaAShort + kDmaB);
 
 __device__ inline void lds_dma16(const void* g, uint8_t* lds) {
   __builtin_amdgcn_global_load_lds(g, (lds_void_t*)lds, 16, 0, 0);
@@ -530,6 +526,20 @@ struct DmaW {
   static constexpr int kRowB = WF == kWfQ8Rows ? kDmaRowB : WF == kWfQ8Pack ? kPackRowB : kPackRowQ4B;
   static constexpr int kInst = (WF == kWfQ8Rows ? kDmaB : 256 * kRowB) / 1024;  // 1 KiB instructions per tile
   static constexpr int64_t kStride = WF == kWfQ8Rows ? 68 : 256 * kRowB;         // global bytes per K tile
+};
+// The LDS ring: three stages for 256-row tiles. Short tiles of the packs take half a CU's LDS (Q8_0 three stages of
+// 25 KiB, Q4_K four of 18), so that a CU holds two blocks: the tile table, permutation and first tiles of one
+// arrive and its rows are stored while the other multiplies. One block with five stages, four tiles in flight, left
+// the CU waiting at both ends of a tile of few K tiles: Qwen-shaped T = 48 146 -> 121 us, d 4096, d_ff 1536, E 128
+// T = 40 408 -> 335, Mixtral-shaped Q4_K T = 12 233 -> 215, Q8_0 T = 13 290 -> 283. The ggml rows' stages (28 KiB, two
+// would fit) keep five.
+template <int WF, bool SHORT>
+struct DmaRing {
+  static constexpr int kA = SHORT ? kDmaAShort : kDmaA;
+  static constexpr int kStage = kA + 1024 * DmaW<WF>::kInst;
+  static constexpr int kStages = !SHORT ? 3 : WF == kWfQ4Pack ? 4 : WF == kWfQ8Pack ? 3 : 5;
+  static constexpr size_t kLds = (size_t)kStages * kStage;
+  static constexpr int kBlocks = kLds + 2048 <= 80 * 1024 ? 2 : 1;  // blocks a CU holds
 };
 
 // The B fragment of K step KS (compile time) from one weight row's K tile in LDS: the lane's 8 elements
@@ -620,16 +630,16 @@ __device__ inline half8 decode_b(const RawB<WF>& r) {
 }
 
 // TAIL (gated only): the launch carries a tail split (gated_item); the other instantiation is the plain
-// XCD-balanced mapping. SHORT: the launch has at most 64 tokens (kDmaStagesShort).
+// XCD-balanced mapping. SHORT: the tiles hold at most 64 rows (DmaRing).
 template <bool GATED, int WF, bool TAIL = false, bool SHORT = false>
-__global__ void __launch_bounds__(kDmaThreads) gemm_dma_q8_kernel(GemmArgs g, int NT) {
+__global__ void __launch_bounds__(kDmaThreads, (2 * DmaRing<WF, SHORT>::kBlocks)) gemm_dma_q8_kernel(GemmArgs g, int NT) {
   constexpr int BN = GATED ? 128 : 256;
   constexpr int kRowB = DmaW<WF>::kRowB;       // LDS bytes per weight row
   constexpr int kLastB = DmaW<WF>::kInst - 1;  // last weight DMA instruction
   constexpr int kDmaInstB = (DmaW<WF>::kInst + 7) / 8;  // weight DMA instructions per wave (the last shared)
-  constexpr int NS = SHORT ? kDmaStagesShort : kDmaStages;  // LDS stages
-  constexpr int kAB = SHORT ? kDmaAShort : kDmaA;           // activation bytes per stage
-  constexpr int kStage = kAB + kDmaB;
+  constexpr int NS = DmaRing<WF, SHORT>::kStages;  // LDS stages
+  constexpr int kAB = DmaRing<WF, SHORT>::kA;      // activation bytes per stage
+  constexpr int kStage = DmaRing<WF, SHORT>::kStage;
   constexpr int kInstA = kAB / 1024 / 8;                    // activation DMA instructions per wave (1 or 4)
   constexpr int kInstMax = kInstA > kDmaInstB ? kInstA : kDmaInstB;
   constexpr int kDmaInst = kInstA + kDmaInstB;
@@ -1543,9 +1553,17 @@ bool gemm_supported(int type, int K) {
          K % GBK == 0;
 }
 
+// EMBER_GEMM_SHORT=0 (read per call): the three-stage kernel anyway, whose outputs the short one matches bit for bit.
+bool short_enabled() {
+  const char* v = std::getenv("EMBER_GEMM_SHORT");
+  return !(v && atoi(v) == 0);
+}
+
 int gemm_max_tiles(int T, int k, int E) { return (T * k + GBM - 1) / GBM + std::min(E, T * k); }
 
-// One 256-token-tile DMA block per CU (its LDS ring takes more than half a CU's LDS).
+// Blocks of the 256-token-tile DMA launches that a round counts: one per CU, whose LDS ring takes more than half a
+// CU's LDS. The packs' short ring fits two, but counting two changed nothing beyond noise where K is split: Mixtral-
+// shaped Q8_0 T = 13 283 / 288 us with two, Q4_K T = 12 207 / 203.
 int gemm_slots() { return device_cus() / 8 * 8; }
 
 // Up to 8 parts and K / 64 (a K tile per part), while the partials (parts x rows x 2N floats) stay within
@@ -1566,22 +1584,18 @@ int gemm_tail_parts(int type, bool packed, int rows, int N, int K) {
 // One DMA tile launch: the weight format's instantiation (Q4_K pack, Q8_0 pack, Q8_0 rows), its LDS.
 template <bool GATED, bool TAIL, bool SHORT>
 int launch_dma(int type, const GemmArgs& gk, int NT, unsigned nb, hipStream_t st) {
-  constexpr size_t lds = SHORT ? kDmaLdsShort : kDmaLds;
-  static const bool ok =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_q8_kernel<GATED, kWfQ8Rows, TAIL, SHORT>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_q8_kernel<GATED, kWfQ8Pack, TAIL, SHORT>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_q8_kernel<GATED, kWfQ4Pack, TAIL, SHORT>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-  if (!ok) return EMBER_ERR_LAUNCH;
-  if (type == EMBER_TYPE_Q4_K)
-    gemm_dma_q8_kernel<GATED, kWfQ4Pack, TAIL, SHORT><<<nb, kDmaThreads, lds, st>>>(gk, NT);
-  else if (gk.Wp)
-    gemm_dma_q8_kernel<GATED, kWfQ8Pack, TAIL, SHORT><<<nb, kDmaThreads, lds, st>>>(gk, NT);
-  else
-    gemm_dma_q8_kernel<GATED, kWfQ8Rows, TAIL, SHORT><<<nb, kDmaThreads, lds, st>>>(gk, NT);
-  return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
+  auto launch = [&](auto WFc) {
+    constexpr int WF = decltype(WFc)::value;
+    constexpr size_t lds = DmaRing<WF, SHORT>::kLds;
+    static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_q8_kernel<GATED, WF, TAIL, SHORT>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+    if (!ok) return EMBER_ERR_LAUNCH;
+    gemm_dma_q8_kernel<GATED, WF, TAIL, SHORT><<<nb, kDmaThreads, lds, st>>>(gk, NT);
+    return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
+  };
+  if (type == EMBER_TYPE_Q4_K) return launch(std::integral_constant<int, kWfQ4Pack>{});
+  if (gk.Wp) return launch(std::integral_constant<int, kWfQ8Pack>{});
+  return launch(std::integral_constant<int, kWfQ8Rows>{});
 }
 
 template <int FMT, bool GATED>
@@ -1608,10 +1622,8 @@ int launch_gemm_fmt(const GemmArgs& g, int max_mtiles, hipStream_t st) {
     unsigned nb = blocks * (unsigned)gk.ksplit;
     // with a tail split: every whole round plus one round of tail parts, whatever the device-side tile count
     if (tail) nb = std::max(nb, (unsigned)((max_mtiles * NT / gk.slots + 1) * gk.slots));
-    // at most 64 tokens: no tile holds more than 64 rows (EMBER_GEMM_SHORT=0, read per call: the
-    // three-stage kernel anyway, whose outputs the short one matches bit for bit)
-    const char* sv = std::getenv("EMBER_GEMM_SHORT");
-    const bool shrt = g.T <= kShortRows && !(sv && atoi(sv) == 0);
+    // at most 64 tokens, or tiles that the dispatch cut at 64 rows
+    const bool shrt = g.short_tiles || (g.T <= kShortRows && short_enabled());
     int s = EMBER_OK;
     if constexpr (GATED) {
       if (tail)
@@ -1735,6 +1747,24 @@ static double expected_row_tiles(int T, int k, int E, int bm) {
   return E * per_e;
 }
 
+// Whether a batch of more than 64 tokens (a smaller one has no longer segment: a token picks an expert once) takes
+// routed tiles of at most 64 rows, and with them the short ring's two blocks per CU. 64- / 256-row tiles, us:
+// - up to 58 (Q4_K) or 40 (Q8_0) mean rows per expert, while a second tile, which reads its weights again, is rare:
+//   Qwen-shaped Q4_K T = 80 124 / 161, T = 512 (32) 159 / 198; Q8_0 T = 256 174 / 202, T = 600 (37) 208 / 236; d 4096,
+//   d_ff 1536, E 128 Q4_K T = 800 (50) 521 / 594, T = 1000 (62) 616 / 647, T = 1200 759 / 725; Mixtral-shaped Q4_K T =
+//   72 223 / 271, T = 220 (55) 316 / 352, T = 240 352 / 354, T = 320 472 / 402, Q8_0 T = 129 (32) 329 / 338, T = 200
+//   (50) 363 / 362, T = 240 425 / 399; DeepSeek-shaped Q8_0 T = 400 (37) 193 / 196, T = 450 204 / 200.
+// - where one 256-row tile of every expert would leave CUs idle, from 52 rows on (below, the batch is one tile an
+//   expert either way), up to 2.5 blocks of 256-row tiles per CU: d 1024, d_ff 2816, E 8 Q8_0 T = 160 (40) 70 / 67, T =
+//   240 (60) 71 / 81, T = 400 80 / 98, T = 1024 118 / 145, T = 2700 (2.1 blocks) 199 / 220, T = 3300 (2.6) 230 / 233,
+//   T = 4096 284 / 275.
+bool gemm_short_tiles(int type, bool packed, int T, int k, int E, int d_ff) {
+  if (T <= kShortRows || !packed || !dma_path(type, packed) || !short_enabled()) return false;
+  const double m = (double)T * k / E, nt = (d_ff + 127) / 128, cus = std::max(1, device_cus());
+  if (E * nt < cus) return m > 52.0 && expected_row_tiles(T, k, E, GBM) * nt <= 2.5 * cus;
+  return m <= (type == EMBER_TYPE_Q4_K ? 58.0 : 40.0);
+}
+
 int gemm_expected_tiles(int T, int k, int E) { return (int)std::ceil(expected_row_tiles(T, k, E, SBM)); }
 
 int gemm_ksplit(int type, bool packed, int T, int k, int E, int N, int K) {
@@ -1748,7 +1778,8 @@ int gemm_ksplit(int type, bool packed, int T, int k, int E, int N, int K) {
   // Binomial(T k, 1 / E) make E[ceil(n / 256)] tiles; normal approximation) times the n-tiles.
   // Mixtral-shaped down projection (K = 14336), ks 1 / 2 / 4, one box: T = 768 814 / 748 / 769 us,
   // T = 1024 1020 / 1047 / 1017 (about half the experts take a second, short tile), T = 8 - / 278 / 282.
-  const double tiles = expected_row_tiles(T, k, E, GBM) * ((N + 255) / 256);
+  const bool shrt = gemm_short_tiles(type, packed, T, k, E, K);
+  const double tiles = expected_row_tiles(T, k, E, shrt ? kShortRows : GBM) * ((N + 255) / 256);
   const double slots = std::max(1, gemm_slots());
   auto rounds = [&](int ks) { return std::ceil(tiles * ks / slots - 1e-6); };  // (a whole count stays whole)
   int best = 1;

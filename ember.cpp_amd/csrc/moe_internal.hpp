@@ -237,6 +237,7 @@ struct GemmArgs {
   const int4* tiles;
   const int32_t* n_tiles;
   const int32_t* xcd;      // DispatchScratch::xcd, or null
+  bool short_tiles;        // 256-token path: the tiles hold at most 64 rows (gemm_short_tiles)
   _Float16* out_h;         // gated: silu(gate) * up as fp16 [pos][N]
   float* out_y;            // plain: f32 [pos][N]
   int ksplit;              // plain projections: K split over this many blocks, partial sums to
@@ -358,6 +359,7 @@ int launch_prefill_pack(int type, const void* W0, const void* W1, int64_t expert
                         int N, int K, uint8_t* dst, hipStream_t st);
 bool gemm_supported(int type, int K);
 int gemm_max_tiles(int T, int k, int E);
+bool gemm_short_tiles(int type, bool packed, int T, int k, int E, int d_ff);
 int launch_gemm(const GemmArgs& g, bool gated, int max_mtiles, hipStream_t st);
 // The activation conversion (ActConv) as a launch of its own: one block per row.
 int launch_act_conv(const ActConv& c, hipStream_t st);

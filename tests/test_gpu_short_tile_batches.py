@@ -1,0 +1,63 @@
+"""Batches of more than 64 tokens on the prefill packs' 64-row tiles (the 256-token path's short ring), chosen by
+the mean rows per expert. The tiles multiply the same fragments in the same order as the 256-row ones
+(EMBER_GEMM_SHORT=0): bit-identical outputs, held to the oracle (utils.cpp:704-748) at the 2e-3 rel-L2 bar of
+the FP16 tiles."""
+import numpy as np
+import pytest
+
+import ember_moe as em
+from gpu_util import rel_l2, run_oracle, same_bits
+
+
+def _layer(kw, pack=True):
+    import torch
+
+    spec = em.LayerSpec(seed=67, **kw)
+    hl = em.make_host_layer(spec)
+    dl = em.DeviceLayer.upload(hl)
+    if pack:
+        buf = torch.empty(em.prefill_pack_bytes(dl.desc), dtype=torch.uint8, device="cuda")
+        em.prefill_pack(dl.desc, buf)
+        dl.tensors["pack"] = buf
+    return spec, hl, dl
+
+
+def _run(dl, x):
+    import torch
+
+    out, _ = dl.forward(torch.from_numpy(np.ascontiguousarray(x)).cuda())
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+WIDE = dict(d=512, d_ff=512, E=64, k=2)  # 64 experts x 4 column tiles: a block for every CU
+FEW = dict(d=512, d_ff=768, E=4, k=2)
+CASES = {
+    # name: (spec kwargs, T): T k / E mean rows, the rule's ends and segments past 64 rows
+    "q8_first": (dict(WIDE, wtype=em.Q8_0), 65),
+    "q8_last": (dict(WIDE, wtype=em.Q8_0), 1280),
+    "q8_past": (dict(WIDE, wtype=em.Q8_0), 1281),
+    "q4_last": (dict(WIDE, wtype=em.Q4_K), 1856),
+    "q4_past": (dict(WIDE, wtype=em.Q4_K), 1857),
+    "few_below": (dict(FEW, wtype=em.Q8_0), 104),
+    "few_first": (dict(FEW, wtype=em.Q8_0), 105),
+    "few_q4": (dict(FEW, wtype=em.Q4_K), 777),
+    "all_on_one": (dict(d=512, d_ff=512, E=64, k=1, wtype=em.Q8_0, bias_std=50.0), 193),
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_short_tiles_of_batches_same_bits(gpu, monkeypatch, name):
+    kw, T = CASES[name]
+    spec, hl, dl = _layer(kw)
+    x = em.make_input(spec, T, seed=68)
+    monkeypatch.setenv("EMBER_MOE_PATH", "gemm")
+    monkeypatch.setenv("EMBER_TAIL_PARTS", "1")
+    print(f"short tiles of a batch {name} T={T}", flush=True)
+    y = _run(dl, x)
+    monkeypatch.setenv("EMBER_GEMM_SHORT", "0")
+    assert same_bits(y, _run(dl, x))
+    err = rel_l2(y, run_oracle(hl, x))
+    print(f"  rel-L2 vs oracle {err:.2e}", flush=True)
+    assert err < 2e-3, err
