@@ -28,7 +28,7 @@ constexpr int kMaxK = 64;   // picks live in a 64-entry LDS array per wave
 enum PathMode { kGemv = 0, kSkinny = 1, kGemm = 2 };
 bool f32_stacks(int type_in, int type_out) { return type_in == EMBER_TYPE_F32 && type_out == EMBER_TYPE_F32; }
 int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int E, bool packed = false,
-              bool with_shared = false) {
+              bool with_shared = false, bool dense = false) {
   const bool f32 = f32_stacks(type_in, type_out);  // tiles on the FP32 matrix cores (moe_gemm_f32.hip)
   if (!f32 && (!gemm_supported(type_in, K_in) || !gemm_supported(type_out, K_out))) return kGemv;
   // tuning override: gemv | skinny | gemm (read per call, so a test can select each kernel); the shared
@@ -47,7 +47,7 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
   // / 335 / 305, T = 8 382 / 335 / 308, T = 12 531 / 341 / 311; T = 32 361 vs 387 us on the 64-token
   // tiles. Without it, GEMV / 256-token tiles: T = 6 345 / 403, T = 8 386 / 404, T = 10 458 / 410)
   const bool q8 = type_in == EMBER_TYPE_Q8_0 && type_out == EMBER_TYPE_Q8_0;
-  if (q8) return avg_m <= (packed ? 1.0 : 2.0) ? kGemv : kGemm;
+  if (q8 && !dense) return avg_m <= (packed ? 1.0 : 2.0) ? kGemv : kGemm;
   // (packed BF16: row exponents for the fp16 MFMA path, which both tile kernels have; without them BF16 runs
   // the split bf16 MFMA, which only the 64-token-tile kernel implements)
   // The expected tokens per expert HIT, T*k / (E (1 - (1 - 1/E)^(T*k))): the GEMV's cost follows the
@@ -86,7 +86,10 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
     return kGemv;
   }
   // (one dense matrix, the shared expert: the 64-token tiles, split over K, up to 800 rows; DeepSeek-shaped layer,
-  // 64- / 256-token tiles: BF16 T = 700 270 / 293 us, T = 850 353 / 302; F16 T = 850 376 / 379, T = 1000 406 / 403)
+  // 64- / 256-token tiles: BF16 T = 700 270 / 293 us, T = 850 353 / 302; F16 T = 850 376 / 379, T = 1000 406 / 403;
+  // Q8_0, whose 256-token tiles kept 22 of the chip's CUs busy for longer than all its routed launches, up to 1600:
+  // T = 12 92 / 120, T = 32 96 / 133, T = 100 105 / 154, T = 200 148 / 191, T = 700 230 / 270, T = 1280 328 / 336, T =
+  // 1536 368 / 401, T = 1800 443 / 405)
   // BF16 (packed) and F16 routed experts: the 64-token tiles stream the weights best while most experts fit one,
   // up to 60 rows per expert (Mixtral-shaped BF16 T = 160 (40) 589 / 733, T = 256 (64) 789 / 784, T = 384 976 / 848)
   // and, with 32 experts and more, whose counts spread further, up to 28 (DeepSeek-shaped BF16 T = 256 (24) 182 /
@@ -96,7 +99,7 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
   const double most64 = E * ((K_out + 127) / 128) < 256 ? 250.0 : E >= 32 ? 28.0 : 60.0;
   if (half && (packed || type_in == EMBER_TYPE_F16 || type_out == EMBER_TYPE_F16) && E > 1)
     return avg_m <= most64 ? kSkinny : kGemm;
-  if (avg_m <= (E > 1 ? 96.0 : half ? 800.0 : 1024.0)) return kSkinny;
+  if (avg_m <= (E > 1 ? 96.0 : half ? 800.0 : q8 ? 1600.0 : 1024.0)) return kSkinny;
   if (type_in == EMBER_TYPE_BF16 && type_out == EMBER_TYPE_BF16 && !packed) return kSkinny;
   return kGemm;
 }
@@ -226,6 +229,9 @@ struct Layout {
   RouteLayout r;
   size_t end;
 };
+bool q8_shared(const ember_moe_layer* w) {
+  return w->gate_shared_type == EMBER_TYPE_Q8_0 && w->down_shared_type == EMBER_TYPE_Q8_0;
+}
 // Whether a call may take the one-token slice launch (SliceArgs): one token on the decode path, the
 // fused routing's limits, a Q8_0 or Q4_K prefill pack, no shared expert; unless any_size, also enough
 // slices to give every CU a block (the scratch layout reserves the section whenever the launch can run).
@@ -235,7 +241,8 @@ bool slices_possible(const ember_moe_layer* w, int T, int mode, bool any_size) {
          packable(w) && w->d_ff_shared == 0 && slices_fit(t, w->d, w->d_ff, w->E, w->k, any_size);
 }
 
-Layout layout(const ember_moe_layer* w, int T) {
+// `lean`: at most that many parts in the K splits of a Q8_0 or F32 shared expert, 0 also without the F32 tiles.
+Layout layout_of(const ember_moe_layer* w, int T, int lean) {
   Layout l;
   const size_t slots = (size_t)T * w->k;
   size_t o = 0;
@@ -257,8 +264,9 @@ Layout layout(const ember_moe_layer* w, int T) {
   l.mode = path_mode(w->gate_type, w->d, w->down_type, w->d_ff, (double)T * w->k / w->E, w->E, w->prefill_pack != nullptr,
                      w->d_ff_shared > 0);
   const bool pack_bf16 = w->prefill_pack && bf16_stacks(w);  // row exponents, also the shared expert's if BF16
+  if (!lean && f32_stacks(w->gate_type, w->down_type)) l.mode = kGemv;
   l.mode_shared = w->d_ff_shared > 0 ? path_mode(w->gate_shared_type, w->d, w->down_shared_type, w->d_ff_shared,
-                                                 (double)T, 1, pack_bf16 && bf16_shared(w))
+                                                 (double)T, 1, pack_bf16 && bf16_shared(w), false, true)
                                      : kGemv;
   // a shared expert of the routed experts' types rides in the routed decode launches as one more segment
   // (a few µs), while on its own its T rows make a dense MFMA launch of only d_ff_shared / 128 blocks
@@ -270,13 +278,17 @@ Layout layout(const ember_moe_layer* w, int T) {
   // (down) blocks per 64 tokens: split over K until the chip is filled (C4 shape, T = 16: 128 -> 25 us)
   l.ks_sh_gu = l.ks_sh_dn = 1;
   const bool f32_sh = w->d_ff_shared > 0 && f32_stacks(w->gate_shared_type, w->down_shared_type);
+  if (!lean && f32_sh) l.mode_shared = kGemv;
+  const int cap = f32_sh || q8_shared(w) ? std::max(1, lean) : kMaxDenseKSplit;
   if (w->d_ff_shared > 0 && l.mode_shared == kSkinny && f32_sh) {
-    l.ks_sh_dn = gemm_f32_ksplit((T + 63) / 64, w->d, w->d_ff_shared);
+    l.ks_sh_dn = std::min(cap, gemm_f32_ksplit((T + 63) / 64, w->d, w->d_ff_shared));
   } else if (w->d_ff_shared > 0 && l.mode_shared == kSkinny) {
     l.ks_sh_gu = gemm_dense_ksplit(true, T, w->d_ff_shared, w->d,
                                    2 * (int64_t)w->d_ff_shared * row_bytes(w->gate_shared_type, w->d));
     l.ks_sh_dn = gemm_dense_ksplit(false, T, w->d, w->d_ff_shared,
                                    (int64_t)w->d * row_bytes(w->down_shared_type, w->d_ff_shared));
+    l.ks_sh_gu = std::min(cap, l.ks_sh_gu);
+    l.ks_sh_dn = std::min(cap, l.ks_sh_dn);
   }
   l.ys = o; o = align_up(o + (w->d_ff_shared > 0 ? (size_t)l.ks_sh_dn * T * w->d * 4 : 0));
   l.shpart = o; o = align_up(o + (l.ks_sh_gu > 1 ? (size_t)l.ks_sh_gu * T * 2 * w->d_ff_shared * 4 : 0));
@@ -298,7 +310,9 @@ Layout layout(const ember_moe_layer* w, int T) {
   l.hexp = o; o = align_up(o + (mfma && !sp ? slots * 4 : 0));
   l.hs16 = o; o = align_up(o + (mfma_sh ? (size_t)T * w->d_ff_shared * (sp_sh ? 4 : 2) : 0));
   l.hsexp = o; o = align_up(o + (mfma_sh && !sp_sh ? (size_t)T * 4 : 0));
-  l.tiles = o; o = align_up(o + (size_t)l.mtiles * 16);
+  // the fp16 and bf16 tiles leave the section h free (h16): at most 17 bytes of its 4 d_ff per slot
+  l.tiles = mfma ? l.h : o;
+  o = align_up(o + (mfma ? 0 : (size_t)l.mtiles * 16));
   // the routed gate/up's tail split (256-token tiles): raw partial gate / up dots [parts][T k][2 d_ff]
   l.tail_parts = l.mode == kGemm ? gemm_tail_parts(w->gate_type, w->prefill_pack != nullptr && !pack_bf16,
                                                    (int)slots, w->d_ff, w->d)
@@ -309,6 +323,20 @@ Layout layout(const ember_moe_layer* w, int T) {
   l.part = o; o = align_up(o + (slices_possible(w, T, l.mode, true) ? (size_t)w->k * (w->d_ff / 64) * w->d * 4 : 0));
   l.end = o;
   return l;
+}
+
+// The scratch of a call. The K splits of a Q8_0 or F32 shared expert and the F32 tile table give way where the
+// call would otherwise miss the allocation-free entry point's buffer by them.
+Layout layout(const ember_moe_layer* w, int T) {
+  const Layout l = layout_of(w, T, kMaxDenseKSplit);
+  const size_t limit = EMBER_MOE_NOALLOC_SCRATCH_BYTES;
+  const bool f32_tiles = l.mode != kGemv && f32_stacks(w->gate_type, w->down_type);
+  if (l.end <= limit || !(f32_tiles || (l.mode_shared == kSkinny && l.ks_sh_gu * l.ks_sh_dn > 1))) return l;
+  if (layout_of(w, T, 0).end > limit) return l;
+  for (int lean = kMaxDenseKSplit / 2;; lean /= 2) {
+    const Layout m = layout_of(w, T, lean);
+    if (m.end <= limit || !lean) return m;
+  }
 }
 
 // The launch plan of a call (which kernels run), shared by run_ffn and ember_moe_path.

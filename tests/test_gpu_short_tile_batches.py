@@ -1,7 +1,10 @@
 """Batches of more than 64 tokens on the prefill packs' 64-row tiles (the 256-token path's short ring), chosen by
-the mean rows per expert. The tiles multiply the same fragments in the same order as the 256-row ones
-(EMBER_GEMM_SHORT=0): bit-identical outputs, held to the oracle (utils.cpp:704-748) at the 2e-3 rel-L2 bar of
-the FP16 tiles."""
+the mean rows per expert, and a Q8_0 shared expert's batch on the dense 64-token tiles, split over K. The routed
+tiles multiply the same fragments in the same order as the 256-row ones (EMBER_GEMM_SHORT=0): bit-identical
+outputs. The shared expert's K split changes the order of its FP32 sums: sqrt(K) 2^-24 = 3e-6 at most for K <= 2048, which
+moves a share of up to 3e-6 / 2^-11 of the hidden values to the next FP16 value, 2^-10 away: sqrt(6e-3) 2^-10 = 8e-5
+rel-L2 against the 256-row tiles. Both are held to the oracle (utils.cpp:704-748) at the 2e-3 rel-L2 bar of the FP16
+tiles."""
 import numpy as np
 import pytest
 
@@ -61,3 +64,35 @@ def test_short_tiles_of_batches_same_bits(gpu, monkeypatch, name):
     err = rel_l2(y, run_oracle(hl, x))
     print(f"  rel-L2 vs oracle {err:.2e}", flush=True)
     assert err < 2e-3, err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [9, 65, 200])
+def test_q8_shared_expert_on_dense_tiles(gpu, monkeypatch, T):
+    spec, hl, dl = _layer(dict(d=512, d_ff=512, E=8, k=2, wtype=em.Q8_0, d_ff_shared=1984), pack=False)
+    x = em.make_input(spec, T, seed=69)
+    print(f"Q8_0 shared expert T={T}", flush=True)
+    y = _run(dl, x)
+    monkeypatch.setenv("EMBER_MOE_SHARED_PATH", "skinny")
+    assert same_bits(y, _run(dl, x))  # the path it takes by itself
+    monkeypatch.setenv("EMBER_MOE_SHARED_PATH", "gemm")
+    assert rel_l2(y, _run(dl, x)) < 1e-4
+    err = rel_l2(y, run_oracle(hl, x))
+    assert err < 2e-3, err
+
+
+@pytest.mark.parametrize("kw,T", [
+    (dict(d=2048, d_ff=1408, E=64, k=6, wtype=em.Q8_0, d_ff_shared=2816), 120),  # 33.2 MB without the K split's parts
+    (dict(d=64, d_ff=64, E=8, k=4, wtype=em.F32), 6412),  # 4 KiB below the buffer's size without the tile table
+])
+def test_scratch_stays_within_the_no_allocation_buffer(kw, T):
+    spec = em.LayerSpec(**kw)
+    L = em.Layer()
+    for n, v in dict(d=spec.d, d_ff=spec.d_ff, E=spec.E, k=spec.k, d_ff_shared=spec.d_ff_shared).items():
+        setattr(L, n, v)
+    sh = ("gate_shared", "up_shared", "down_shared") if spec.d_ff_shared else ()
+    for n in ("gate", "up", "down") + sh:
+        setattr(L, n, 1 << 20)  # (never read)
+        setattr(L, n.split("_")[0] + ("_shared_type" if "_" in n else "_type"), spec.wtype)
+    L.router = 1 << 20
+    assert 0 < em.scratch_bytes(L, T) <= 32 << 20
