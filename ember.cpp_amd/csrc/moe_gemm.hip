@@ -1758,6 +1758,8 @@ static double expected_row_tiles(int T, int k, int E, int bm) {
 //   expert either way), up to 2.5 blocks of 256-row tiles per CU: d 1024, d_ff 2816, E 8 Q8_0 T = 160 (40) 70 / 67, T =
 //   240 (60) 71 / 81, T = 400 80 / 98, T = 1024 118 / 145, T = 2700 (2.1 blocks) 199 / 220, T = 3300 (2.6) 230 / 233,
 //   T = 4096 284 / 275.
+// The ggml rows keep 256-row tiles, since their short ring leaves one block per CU (Mixtral-shaped Q8_0 T = 129 439 /
+// 440, T = 150 460 / 449; DeepSeek-shaped T = 400 230 / 191).
 bool gemm_short_tiles(int type, bool packed, int T, int k, int E, int d_ff) {
   if (T <= kShortRows || !packed || !dma_path(type, packed) || !short_enabled()) return false;
   const double m = (double)T * k / E, nt = (d_ff + 127) / 128, cus = std::max(1, device_cus());
