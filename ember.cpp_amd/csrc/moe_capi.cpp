@@ -449,7 +449,22 @@ const char* ember_moe_strerror(int status) {
 
 size_t ember_moe_scratch_bytes(const ember_moe_layer* w, int T) {
   if (validate(w) != EMBER_OK || T < 0) return 0;
-  return layout(w, std::max(T, 1)).end;
+  T = std::max(T, 1);
+  const size_t end = layout(w, T).end, limit = EMBER_MOE_NOALLOC_SCRATCH_BYTES;
+  // A scratch buffer sized for a batch serves the smaller ones too, although a Q8_0 or F32 shared expert's K split,
+  // and with it the parts' sections, shrinks as the rows grow: room for any smaller batch's parts (the dense split
+  // keeps them within the weights' bytes, the F32 one within four), while a call of the allocation-free entry
+  // point stays one (layout keeps the smaller ones within its buffer then).
+  size_t extra = 0;
+  if (w->d_ff_shared > 0 && q8_shared(w) && T > 2)
+    extra = (size_t)w->d_ff_shared * 2 * row_bytes(EMBER_TYPE_Q8_0, w->d) +
+            (size_t)w->d * row_bytes(EMBER_TYPE_Q8_0, w->d_ff_shared) + 512;
+  else if (w->d_ff_shared > 0 && f32_stacks(w->gate_shared_type, w->down_shared_type) && T > 64)
+    extra = (size_t)T * w->d * 4 * (kMaxKSplit - 1) + 256;
+  else if (!f32_stacks(w->gate_type, w->down_type))
+    return end;
+  const size_t size = std::max(end, layout_of(w, T, 1).end + extra);
+  return end <= limit ? std::min(size, limit) : size;
 }
 
 namespace {

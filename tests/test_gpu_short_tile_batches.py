@@ -81,11 +81,7 @@ def test_q8_shared_expert_on_dense_tiles(gpu, monkeypatch, T):
     assert err < 2e-3, err
 
 
-@pytest.mark.parametrize("kw,T", [
-    (dict(d=2048, d_ff=1408, E=64, k=6, wtype=em.Q8_0, d_ff_shared=2816), 120),  # 33.2 MB without the K split's parts
-    (dict(d=64, d_ff=64, E=8, k=4, wtype=em.F32), 6412),  # 4 KiB below the buffer's size without the tile table
-])
-def test_scratch_stays_within_the_no_allocation_buffer(kw, T):
+def _desc(kw):
     spec = em.LayerSpec(**kw)
     L = em.Layer()
     for n, v in dict(d=spec.d, d_ff=spec.d_ff, E=spec.E, k=spec.k, d_ff_shared=spec.d_ff_shared).items():
@@ -95,4 +91,22 @@ def test_scratch_stays_within_the_no_allocation_buffer(kw, T):
         setattr(L, n, 1 << 20)  # (never read)
         setattr(L, n.split("_")[0] + ("_shared_type" if "_" in n else "_type"), spec.wtype)
     L.router = 1 << 20
-    assert 0 < em.scratch_bytes(L, T) <= 32 << 20
+    return L
+
+
+@pytest.mark.parametrize("kw,T", [
+    (dict(d=2048, d_ff=1408, E=64, k=6, wtype=em.Q8_0, d_ff_shared=2816), 120),  # 33.2 MB without the K split's parts
+    (dict(d=64, d_ff=64, E=8, k=4, wtype=em.F32), 6412),  # 4 KiB below the buffer's size without the tile table
+])
+def test_scratch_stays_within_the_no_allocation_buffer(kw, T):
+    assert 0 < em.scratch_bytes(_desc(kw), T) <= 32 << 20
+
+
+@pytest.mark.parametrize("kw,Ts", [
+    (dict(d=2048, d_ff=1408, E=64, k=6, wtype=em.Q8_0, d_ff_shared=2816), range(1, 200)),
+    (dict(d=512, d_ff=512, E=16, k=2, wtype=em.F32, d_ff_shared=2048), range(1, 1200, 7)),
+])
+def test_scratch_of_a_batch_serves_smaller_ones(kw, Ts):
+    L = _desc(kw)
+    sizes = [em.scratch_bytes(L, T) for T in Ts]
+    assert sizes == sorted(sizes)
