@@ -18,7 +18,8 @@
 // roundings deep than the GEMV at any K (layer error against 64 bits 1.6e-7 to 1.7e-7, the GEMV's 1.6e-7 to
 // 2.0e-7). The additions are not hidden (FP32 MFMAs and FP32 VALU instructions do not overlap on gfx950: 4 of
 // each take the sum of their times, and the counters put this kernel's MFMA and VALU cycles together at 93 %
-// of its time): 11 of them per 64 columns and output, a third of the MFMA time.
+// of its time): 11 of them per 64 columns and output, a third of the MFMA time,
+// and a twelfth instruction that keeps infinite sums infinite.
 #include <cstdlib>
 #include <type_traits>
 
@@ -152,11 +153,17 @@ __global__ void __launch_bounds__(kF32Threads, 3) gemm_f32_kernel(GemmF32Args g,
 #pragma unroll
     for (int r = 0; r < 16; ++r) mid[r] = first ? c0[r] + c1[r] : mid[r] + (c0[r] + c1[r]);
   };
-  auto fold = [&] {  // sum += mid + the pair's last two chains, compensated
+  // sum += mid + the pair's last two chains, compensated. The compensation of an infinite sum would be Inf - Inf: the
+  // clamp (v_med3, whose result for a NaN is its lower bound) keeps it finite and too small to carry a finite v past
+  // the largest float, so that an infinite sum stays one, as in the GEMV; it cuts real ones from sums of 2^125 on only
+  // (d 1024, d_ff 2816, E 8, 400 tokens 218.7 -> 221.3 us; running the sums of a block with a NaN again without the
+  // compensation, 220.4, would keep a second copy of the loop).
+  constexpr float kMostComp = 0x1p100f;
+  auto fold = [&] {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const float v = (mid[r] + (c0[r] + c1[r])) - comp[r], t = sum[r] + v;
-      comp[r] = (t - sum[r]) - v;
+      comp[r] = __builtin_amdgcn_fmed3f((t - sum[r]) - v, -kMostComp, kMostComp);
       sum[r] = t;
     }
   };
