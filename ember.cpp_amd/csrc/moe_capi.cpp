@@ -85,7 +85,7 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
   } else if (avg_m <= 2.0) {
     return kGemv;
   }
-  // (one dense matrix, the shared expert: the 64-token tiles, split over K, up to 800 rows; DeepSeek-shaped layer,
+  // (one dense matrix, the shared expert: the 64-token tiles, split over K (Q8_0: the down projection), up to 800 rows; DeepSeek-shaped layer,
   // 64- / 256-token tiles: BF16 T = 700 270 / 293 us, T = 850 353 / 302; F16 T = 850 376 / 379, T = 1000 406 / 403;
   // Q8_0, whose 256-token tiles kept 22 of the chip's CUs busy for longer than all its routed launches, up to 1600:
   // T = 12 92 / 120, T = 32 96 / 133, T = 100 105 / 154, T = 200 148 / 191, T = 700 230 / 270, T = 1280 328 / 336, T =
@@ -283,9 +283,9 @@ Layout layout_of(const ember_moe_layer* w, int T, int lean) {
   if (w->d_ff_shared > 0 && l.mode_shared == kSkinny && f32_sh) {
     l.ks_sh_dn = std::min(cap, gemm_f32_ksplit((T + 63) / 64, w->d, w->d_ff_shared));
   } else if (w->d_ff_shared > 0 && l.mode_shared == kSkinny) {
-    l.ks_sh_gu = gemm_dense_ksplit(true, T, w->d_ff_shared, w->d,
+    l.ks_sh_gu = gemm_dense_ksplit(w->gate_shared_type, true, T, w->d_ff_shared, w->d,
                                    2 * (int64_t)w->d_ff_shared * row_bytes(w->gate_shared_type, w->d));
-    l.ks_sh_dn = gemm_dense_ksplit(false, T, w->d, w->d_ff_shared,
+    l.ks_sh_dn = gemm_dense_ksplit(w->down_shared_type, false, T, w->d, w->d_ff_shared,
                                    (int64_t)w->d * row_bytes(w->down_shared_type, w->d_ff_shared));
     l.ks_sh_gu = std::min(cap, l.ks_sh_gu);
     l.ks_sh_dn = std::min(cap, l.ks_sh_dn);
@@ -457,8 +457,7 @@ size_t ember_moe_scratch_bytes(const ember_moe_layer* w, int T) {
   // point stays one (layout keeps the smaller ones within its buffer then).
   size_t extra = 0;
   if (w->d_ff_shared > 0 && q8_shared(w) && T > 2)
-    extra = (size_t)w->d_ff_shared * 2 * row_bytes(EMBER_TYPE_Q8_0, w->d) +
-            (size_t)w->d * row_bytes(EMBER_TYPE_Q8_0, w->d_ff_shared) + 512;
+    extra = (size_t)w->d * row_bytes(EMBER_TYPE_Q8_0, w->d_ff_shared) + 256;
   else if (w->d_ff_shared > 0 && f32_stacks(w->gate_shared_type, w->down_shared_type) && T > 64)
     extra = (size_t)T * w->d * 4 * (kMaxKSplit - 1) + 256;
   else if (!f32_stacks(w->gate_type, w->down_type))

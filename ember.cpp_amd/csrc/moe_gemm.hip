@@ -1724,7 +1724,8 @@ int launch_gemm_skinny(const GemmArgs& g, bool gated, int max_mtiles, hipStream_
   return gated ? launch_skinny_t<true>(g, max_mtiles, st) : launch_skinny_t<false>(g, max_mtiles, st);
 }
 
-int gemm_dense_ksplit(bool gated, int T, int N, int K, int64_t weight_bytes) {
+int gemm_dense_ksplit(int type, bool gated, int T, int N, int K, int64_t weight_bytes) {
+  if (gated && dma_path(type, false)) return 1;  // gemm_dma64_q8_kernel has no parts of gate / up dots
   const int mt = (T + SBM - 1) / SBM, nt = (N + (gated ? 127 : 255)) / (gated ? 128 : 256), nk = K / GBK;
   const int64_t part_row = (int64_t)T * N * 4 * (gated ? 2 : 1);  // bytes of one part
   int ks = 1;

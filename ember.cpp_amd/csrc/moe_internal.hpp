@@ -375,9 +375,9 @@ constexpr int kMaxKSplit = 4;
 int gemm_skinny_ksplit(int type, bool packed, int T, int k, int E, int N, int K);
 // ... and of a dense projection (the shared expert's T rows) on the 64-token tiles, gated or plain: up to
 // kMaxDenseKSplit parts, until the launch has 512 blocks, each part keeps >= 2 K tiles and the partial
-// sums (f32) stay within the weights' bytes
+// sums (f32) stay within the weights' bytes; 1 for the gated launch of a type the DMA kernels take (Q8_0)
 constexpr int kMaxDenseKSplit = 16;
-int gemm_dense_ksplit(bool gated, int T, int N, int K, int64_t weight_bytes);
+int gemm_dense_ksplit(int type, bool gated, int T, int N, int K, int64_t weight_bytes);
 // ... and of the 256-token-tile path's (the down launch of a long prefill has few blocks per n-tile row)
 int gemm_ksplit(int type, bool packed, int T, int k, int E, int N, int K);
 // Whether the DMA tile kernels serve stacks of `type` (packed: with a prefill pack): Q8_0, packed Q4_K.
