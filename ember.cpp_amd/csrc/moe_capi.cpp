@@ -225,7 +225,9 @@ struct Layout {
   bool short_tiles;                       // the 256-token path's tiles hold at most 64 rows
   int mtiles;                             // most row tiles of the routed launches
   int mode, mode_shared;                  // PathMode of the routed experts and of the shared expert
+  int ksplit;                             // K split of the routed down projection: y's parts in use
   int ks_sh_gu, ks_sh_dn;                 // K split of the shared expert's 64-token-tile launches
+  bool tight;                             // F32 tiles without a section for their table (layout)
   RouteLayout r;
   size_t end;
 };
@@ -241,9 +243,9 @@ bool slices_possible(const ember_moe_layer* w, int T, int mode, bool any_size) {
          packable(w) && w->d_ff_shared == 0 && slices_fit(t, w->d, w->d_ff, w->E, w->k, any_size);
 }
 
-// `lean`: at most that many parts in the K splits of a Q8_0 or F32 shared expert, 0 also without the F32 tiles.
-Layout layout_of(const ember_moe_layer* w, int T, int lean) {
+Layout layout_of(const ember_moe_layer* w, int T, bool tight) {
   Layout l;
+  l.tight = tight;
   const size_t slots = (size_t)T * w->k;
   size_t o = 0;
   l.flag = o; o = align_up(o + (size_t)8 * (2 * w->E + 3));
@@ -264,7 +266,6 @@ Layout layout_of(const ember_moe_layer* w, int T, int lean) {
   l.mode = path_mode(w->gate_type, w->d, w->down_type, w->d_ff, (double)T * w->k / w->E, w->E, w->prefill_pack != nullptr,
                      w->d_ff_shared > 0);
   const bool pack_bf16 = w->prefill_pack && bf16_stacks(w);  // row exponents, also the shared expert's if BF16
-  if (!lean && f32_stacks(w->gate_type, w->down_type)) l.mode = kGemv;
   l.mode_shared = w->d_ff_shared > 0 ? path_mode(w->gate_shared_type, w->d, w->down_shared_type, w->d_ff_shared,
                                                  (double)T, 1, pack_bf16 && bf16_shared(w), false, true)
                                      : kGemv;
@@ -278,27 +279,31 @@ Layout layout_of(const ember_moe_layer* w, int T, int lean) {
   // (down) blocks per 64 tokens: split over K until the chip is filled (C4 shape, T = 16: 128 -> 25 us)
   l.ks_sh_gu = l.ks_sh_dn = 1;
   const bool f32_sh = w->d_ff_shared > 0 && f32_stacks(w->gate_shared_type, w->down_shared_type);
-  if (!lean && f32_sh) l.mode_shared = kGemv;
-  const int cap = f32_sh || q8_shared(w) ? std::max(1, lean) : kMaxDenseKSplit;
   if (w->d_ff_shared > 0 && l.mode_shared == kSkinny && f32_sh) {
-    l.ks_sh_dn = std::min(cap, gemm_f32_ksplit((T + 63) / 64, w->d, w->d_ff_shared));
+    l.ks_sh_dn = gemm_f32_ksplit((T + 63) / 64, w->d, w->d_ff_shared);
   } else if (w->d_ff_shared > 0 && l.mode_shared == kSkinny) {
     l.ks_sh_gu = gemm_dense_ksplit(w->gate_shared_type, true, T, w->d_ff_shared, w->d,
                                    2 * (int64_t)w->d_ff_shared * row_bytes(w->gate_shared_type, w->d));
     l.ks_sh_dn = gemm_dense_ksplit(w->down_shared_type, false, T, w->d, w->d_ff_shared,
                                    (int64_t)w->d * row_bytes(w->down_shared_type, w->d_ff_shared));
-    l.ks_sh_gu = std::min(cap, l.ks_sh_gu);
-    l.ks_sh_dn = std::min(cap, l.ks_sh_dn);
   }
-  l.ys = o; o = align_up(o + (w->d_ff_shared > 0 ? (size_t)l.ks_sh_dn * T * w->d * 4 : 0));
-  l.shpart = o; o = align_up(o + (l.ks_sh_gu > 1 ? (size_t)l.ks_sh_gu * T * 2 * w->d_ff_shared * 4 : 0));
   l.short_tiles = l.mode == kGemm && gemm_short_tiles(w->gate_type, w->prefill_pack != nullptr, T, w->k, w->E, w->d_ff);
   l.mtiles = l.mode == kGemv                      ? 0
              : l.mode == kGemm && !l.short_tiles ? gemm_max_tiles(T, w->k, w->E)
                                                  : gemm_skinny_max_tiles(T, w->k, w->E);
+  const bool f32 = f32_stacks(w->gate_type, w->down_type), packed = w->prefill_pack && !pack_bf16;
+  l.ksplit = l.mode == kGemv      ? 1
+             : f32                ? gemm_f32_ksplit(gemm_expected_tiles(T, w->k, w->E), w->d, w->d_ff)
+             : l.mode == kSkinny ? gemm_skinny_ksplit(w->down_type, packed, T, w->k, w->E, w->d, w->d_ff)
+                                  : gemm_ksplit(w->down_type, packed, T, w->k, w->E, w->d, w->d_ff);
+  // (two parts fewer leave the room that a split of an F32 shared expert and, if tight, the tile table take in y)
+  if (l.mode != kGemv && f32 && (tight || (f32_sh && l.ks_sh_dn > 1))) l.ksplit = std::min(l.ksplit, 2);
   // (the F32 tiles read x and write h in f32: none of the converted activations below)
-  const bool mfma = l.mode != kGemv && !f32_stacks(w->gate_type, w->down_type);
+  const bool mfma = l.mode != kGemv && !f32;
   const bool mfma_sh = w->d_ff_shared > 0 && l.mode_shared != kGemv && !f32_sh;
+  const size_t ys_parts = f32_sh || q8_shared(w) ? 1 : l.ks_sh_dn;
+  l.ys = o; o = align_up(o + (w->d_ff_shared > 0 ? ys_parts * T * w->d * 4 : 0));
+  l.shpart = o; o = align_up(o + (l.ks_sh_gu > 1 ? (size_t)l.ks_sh_gu * T * 2 * w->d_ff_shared * 4 : 0));
   const bool sp = split_bf16(w->gate_type, w->down_type) && !pack_bf16;
   const bool sp_sh = w->d_ff_shared > 0 && split_bf16(w->gate_shared_type, w->down_shared_type) &&
                      !(pack_bf16 && bf16_shared(w));
@@ -310,9 +315,22 @@ Layout layout_of(const ember_moe_layer* w, int T, int lean) {
   l.hexp = o; o = align_up(o + (mfma && !sp ? slots * 4 : 0));
   l.hs16 = o; o = align_up(o + (mfma_sh ? (size_t)T * w->d_ff_shared * (sp_sh ? 4 : 2) : 0));
   l.hsexp = o; o = align_up(o + (mfma_sh && !sp_sh ? (size_t)T * 4 : 0));
-  // the fp16 and bf16 tiles leave the section h free (h16): at most 17 bytes of its 4 d_ff per slot
-  l.tiles = mfma ? l.h : o;
-  o = align_up(o + (mfma ? 0 : (size_t)l.mtiles * 16));
+  // the fp16 and bf16 tiles leave the section h free (h16): the tile table takes at most 17 bytes of its 4 d_ff per
+  // slot. The F32 ones get a section, or, if tight, the end of y, whose last two parts (8 d per slot) are free then.
+  const size_t table = (size_t)l.mtiles * 16, y_part = slots * w->d * 4;
+  l.tiles = mfma ? l.h : tight ? l.y + kMaxKSplit * y_part - table : o;
+  o = align_up(o + (mfma || tight ? 0 : table));
+  // The down parts of a Q8_0 or F32 shared expert take room that the call has in any case, so that no call needs
+  // more scratch by its split: the parts of y that the routed down launch leaves (they run side by side), or h
+  // behind the tile table; as many as fit (DeepSeek-shaped 6 (4 - ksplit) parts in y). The other formats' have a section.
+  const size_t ys_part = (size_t)T * w->d * 4;
+  if (l.ks_sh_dn > 1 && (f32_sh || q8_shared(w))) {
+    const size_t y_room = (kMaxKSplit - l.ksplit) * y_part - (tight ? table : 0);
+    const size_t h_room = mfma ? slots * w->d_ff * 4 - std::min(align_up(table), slots * w->d_ff * 4) : 0;
+    const size_t fit = std::max(y_room, h_room) / ys_part;
+    while (l.ks_sh_dn > 1 && (size_t)l.ks_sh_dn > fit) l.ks_sh_dn /= 2;
+    if (l.ks_sh_dn > 1) l.ys = y_room >= h_room ? l.y + l.ksplit * y_part : l.h + align_up(table);
+  }
   // the routed gate/up's tail split (256-token tiles): raw partial gate / up dots [parts][T k][2 d_ff]
   l.tail_parts = l.mode == kGemm ? gemm_tail_parts(w->gate_type, w->prefill_pack != nullptr && !pack_bf16,
                                                    (int)slots, w->d_ff, w->d)
@@ -325,18 +343,14 @@ Layout layout_of(const ember_moe_layer* w, int T, int lean) {
   return l;
 }
 
-// The scratch of a call. The K splits of a Q8_0 or F32 shared expert and the F32 tile table give way where the
-// call would otherwise miss the allocation-free entry point's buffer by them.
+// The scratch of a call. A call on the F32 tiles that their table (at most 17 bytes per slot) would push past the
+// allocation-free entry point's buffer finds room for it in y, at a K split of at most 2.
 Layout layout(const ember_moe_layer* w, int T) {
-  const Layout l = layout_of(w, T, kMaxDenseKSplit);
+  const Layout l = layout_of(w, T, false);
   const size_t limit = EMBER_MOE_NOALLOC_SCRATCH_BYTES;
-  const bool f32_tiles = l.mode != kGemv && f32_stacks(w->gate_type, w->down_type);
-  if (l.end <= limit || !(f32_tiles || (l.mode_shared == kSkinny && l.ks_sh_gu * l.ks_sh_dn > 1))) return l;
-  if (layout_of(w, T, 0).end > limit) return l;
-  for (int lean = kMaxDenseKSplit / 2;; lean /= 2) {
-    const Layout m = layout_of(w, T, lean);
-    if (m.end <= limit || !lean) return m;
-  }
+  if (l.end <= limit || l.mode == kGemv || !f32_stacks(w->gate_type, w->down_type)) return l;
+  const Layout t = layout_of(w, T, true);
+  return t.end <= limit ? t : l;
 }
 
 // The launch plan of a call (which kernels run), shared by run_ffn and ember_moe_path.
@@ -449,21 +463,8 @@ const char* ember_moe_strerror(int status) {
 
 size_t ember_moe_scratch_bytes(const ember_moe_layer* w, int T) {
   if (validate(w) != EMBER_OK || T < 0) return 0;
-  T = std::max(T, 1);
-  const size_t end = layout(w, T).end, limit = EMBER_MOE_NOALLOC_SCRATCH_BYTES;
-  // A scratch buffer sized for a batch serves the smaller ones too, although a Q8_0 or F32 shared expert's K split,
-  // and with it the parts' sections, shrinks as the rows grow: room for any smaller batch's parts (the dense split
-  // keeps them within the weights' bytes, the F32 one within four), while a call of the allocation-free entry
-  // point stays one (layout keeps the smaller ones within its buffer then).
-  size_t extra = 0;
-  if (w->d_ff_shared > 0 && q8_shared(w) && T > 2)
-    extra = (size_t)w->d * row_bytes(EMBER_TYPE_Q8_0, w->d_ff_shared) + 256;
-  else if (w->d_ff_shared > 0 && f32_stacks(w->gate_shared_type, w->down_shared_type) && T > 64)
-    extra = (size_t)T * w->d * 4 * (kMaxKSplit - 1) + 256;
-  else if (!f32_stacks(w->gate_type, w->down_type))
-    return end;
-  const size_t size = std::max(end, layout_of(w, T, 1).end + extra);
-  return end <= limit ? std::min(size, limit) : size;
+  const Layout l = layout(w, std::max(T, 1));
+  return l.tight ? EMBER_MOE_NOALLOC_SCRATCH_BYTES : l.end;  // (no less than a smaller batch with its table needs)
 }
 
 namespace {
@@ -527,7 +528,6 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
   }
   float* h = at<float>(scratch, l.h);
   float* y = at<float>(scratch, l.y);
-  int ksplit = 1;  // partial sums per y row (K split of the down projection)
 
   const int groups_n = std::max(w->groups_n, 1), groups_top = std::max(w->groups_top, 1);
   const int renorm = w->renorm ? 1 : 0, routed = is_routed(w) ? 1 : 0;
@@ -720,7 +720,7 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     g.N = d;
     g.K = d_ff;
     g.out = y;
-    g.ksplit = ksplit = gemm_f32_ksplit(gemm_expected_tiles(T, k, E), d, d_ff);
+    g.ksplit = l.ksplit;
     g.part_stride = (int64_t)T * k * d;
     if ((s = launch_gemm_f32(g, false, mt, st))) return s;
     mark(ev, 5, st);
@@ -793,8 +793,7 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     g.w_exp0 = pack_bf16 ? wexp(bx.down) : nullptr;
     g.w_exp1 = nullptr;
     g.w_hexp = nullptr;
-    g.ksplit = ksplit = skinny ? gemm_skinny_ksplit(g.type, pack != nullptr, T, k, E, d, d_ff)
-                               : gemm_ksplit(g.type, pack != nullptr, T, k, E, d, d_ff);
+    g.ksplit = l.ksplit;
     g.part_stride = (int64_t)T * k * d;
     if ((s = gemm(g, false, mt))) return s;
     mark(ev, 5, st);
@@ -992,7 +991,7 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
   }
   mark(ev, 6, st);
   const int ys_parts = shared_mfma && l.mode_shared == kSkinny ? l.ks_sh_dn : 1;
-  s = launch_combine(y, ksplit, (int64_t)T * k * d, gates, ds.pos, ys, ys_parts, (int64_t)T * d, sg, out_scale, T, k,
+  s = launch_combine(y, l.ksplit, (int64_t)T * k * d, gates, ds.pos, ys, ys_parts, (int64_t)T * d, sg, out_scale, T, k,
                      d, out, st, fuse_route && !routed ? flag + 2 + 2 * E : nullptr);
   mark(ev, 7, st);
   return s;
