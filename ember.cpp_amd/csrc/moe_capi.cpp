@@ -27,8 +27,10 @@ constexpr int kMaxK = 64;   // picks live in a 64-entry LDS array per wave
 // GEMV, then the FP32 MFMA tiles (64 tokens) at any size.
 enum PathMode { kGemv = 0, kSkinny = 1, kGemm = 2 };
 bool f32_stacks(int type_in, int type_out) { return type_in == EMBER_TYPE_F32 && type_out == EMBER_TYPE_F32; }
-int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int E, bool packed = false,
+// (K_in = d, K_out = d_ff; with_shared: a shared expert, for F32 stacks one of F32 too; dense: the shared expert, E = 1)
+int path_mode(int type_in, int K_in, int type_out, int K_out, int T, int k, int E, bool packed = false,
               bool with_shared = false, bool dense = false) {
+  const double avg_m = (double)T * k / E;
   const bool f32 = f32_stacks(type_in, type_out);  // tiles on the FP32 matrix cores (moe_gemm_f32.hip)
   if (!f32 && (!gemm_supported(type_in, K_in) || !gemm_supported(type_out, K_out))) return kGemv;
   // tuning override: gemv | skinny | gemm (read per call, so a test can select each kernel); the shared
@@ -55,17 +57,27 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, double avg_m, int 
   const double slots = avg_m * E;
   const double hit = slots > 0.0 ? E * (1.0 - std::pow(1.0 - 1.0 / E, slots)) : 0.0;
   const double per_hit = hit > 0.0 ? slots / hit : 0.0;
-  // F32: the GEMV up to 2.6 tokens per hit expert (GEMV / tiles, d 1024, d_ff 2816, E 8: T = 8 (2.3) 92 / 97
-  // us, T = 10 (2.7) 104 / 102, T = 64 322 / 106, T = 400 1719 / 223), up to 2.1 when the layer's stacks exceed 1
-  // GB and a second pass over them costs the most (Mixtral-shaped T = 6 (1.9) 1200 / 1324, T = 8 (2.3) 1445 /
-  // 1351, T = 128 17251 / 1814; Qwen-shaped T = 16 (1.5) 399 / 438, T = 32 (2.3) 614 / 562), up to 3 when they
-  // are under 32 MB and launches and latency set the time (d 256, d_ff 688, E 8: T = 8 (2.3) 33 / 36, T = 12
-  // (3.1) 42 / 41, T = 512 496 / 56). A dense shared expert, whose few tiles leave most CUs idle in a small
-  // batch, up to 64 rows.
+  // F32: the GEMV up to 3 tokens per hit expert (GEMV / tiles, us: d 1024, d_ff 2816, E 8 T = 10 (2.7) 96 / 100, T = 14
+  // (3.6) 113 / 101; d 3072, d_ff 4096, E 16 T = 8 (2.3) 475 / 594, T = 12 (3.1) 670 / 598; d 2048, d_ff 8192, E 16 T =
+  // 20 (2.7) 698 / 808, T = 24 (3.1) 834 / 806; d 512, d_ff 1024, E 16 T = 16 56 / 61, T = 24 67 / 62; top-1 of d
+  // 1024, d_ff 2816, E 8 T = 20 (2.7) 104 / 97), up to 2.1 from 32 experts on, most of which then still have one row
+  // (Qwen-shaped T = 20 (1.8) 459 / 483, T = 32 (2.3) 612 / 553; d 2048, d_ff 768, E 64 T = 12 (1.9) 273 / 283, T =
+  // 16 (2.3) 321 / 314; d 256, d_ff 704, E 32 T = 14 (2.1) 52 / 51), and where one expert's stacks pass the last-level
+  // cache's 256 MB, so that a second pass over them comes from memory (Mixtral-shaped T = 7 (2.1) 1218 / 1304, T = 8 (2.3)
+  // 1430 / 1315, T = 12 1770 / 1316). One matrix, whose few tiles leave most CUs idle in a small batch: up to 18 rows (d
+  // 1024, d_ff 2816 T = 12 75 / 83, T = 16 92 / 83; d 2048, d_ff 8192 T = 16 222 / 235, T = 24 315 / 239; d 4096, d_ff
+  // 14336 T = 8 487 / 632, T = 12 716 / 643).
+  // With an F32 shared expert, which rides in the routed GEMV launches as one more segment but costs two launches of its own
+  // beside the tiles, both take the tiles past 18 tokens and 2.4 per hit expert, from 32 experts on 2.1 (d 1024, d_ff
+  // 768, E 16, d_ff_shared 2048: both GEMV / tiles and GEMV / both tiles T = 12 110 / 134 / 125, T = 16 136 / 147 / 125, T
+  // = 32 229 / 200 / 126; d 512, d_ff 1024, E 16 T = 16 85 / 115 / 94, T = 20 97 / 127 / 95; DeepSeek-shaped T = 20 (2.2)
+  // 343 / 264 / 219; with d_ff_shared 512 T = 20 527 / 622 / 568, T = 24 585 / 637 / 568; E 128, k 2 T = 48 (1.4) 410 / 545 /
+  // 407).
   if (f32) {
-    const int64_t bytes = (int64_t)E * 12 * K_in * K_out;
-    const double most = bytes < ((int64_t)32 << 20) ? 3.0 : bytes > ((int64_t)1 << 30) ? 2.1 : 2.6;
-    return (E == 1 ? avg_m <= 64.0 : per_hit <= most) ? kGemv : kSkinny;
+    if (E == 1) return avg_m <= 18.0 ? kGemv : kSkinny;
+    const bool past_cache = (int64_t)12 * K_in * K_out > ((int64_t)256 << 20);
+    const double most = E >= 32 || past_cache ? 2.1 : with_shared ? 2.4 : 3.0;
+    return per_hit <= most || (with_shared && T <= 18) ? kGemv : kSkinny;
   }
   // packed Q4_K (the same DMA tile kernels): the GEMV up to 1.55 tokens per hit expert, then the
   // 256-token tiles (Qwen-shaped E = 128, GEMV / 64-token / 256-token tiles: T = 13 (1.47) 114 / 119 / 116
@@ -263,11 +275,12 @@ Layout layout_of(const ember_moe_layer* w, int T, bool tight) {
   l.y = o; o = align_up(o + slots * w->d * 4 * kMaxKSplit);
   l.hs = o; o = align_up(o + (size_t)T * w->d_ff_shared * 4);
   l.sg = o; o = align_up(o + (w->shared_gate ? (size_t)T * 4 : 0));
-  l.mode = path_mode(w->gate_type, w->d, w->down_type, w->d_ff, (double)T * w->k / w->E, w->E, w->prefill_pack != nullptr,
-                     w->d_ff_shared > 0);
+  const bool f32_sh = w->d_ff_shared > 0 && f32_stacks(w->gate_shared_type, w->down_shared_type);
+  l.mode = path_mode(w->gate_type, w->d, w->down_type, w->d_ff, T, w->k, w->E, w->prefill_pack != nullptr,
+                     f32_stacks(w->gate_type, w->down_type) ? f32_sh : w->d_ff_shared > 0);
   const bool pack_bf16 = w->prefill_pack && bf16_stacks(w);  // row exponents, also the shared expert's if BF16
   l.mode_shared = w->d_ff_shared > 0 ? path_mode(w->gate_shared_type, w->d, w->down_shared_type, w->d_ff_shared,
-                                                 (double)T, 1, pack_bf16 && bf16_shared(w), false, true)
+                                                 T, 1, 1, pack_bf16 && bf16_shared(w), false, true)
                                      : kGemv;
   // a shared expert of the routed experts' types rides in the routed decode launches as one more segment
   // (a few µs), while on its own its T rows make a dense MFMA launch of only d_ff_shared / 128 blocks
@@ -278,7 +291,6 @@ Layout layout_of(const ember_moe_layer* w, int T, bool tight) {
   // the shared expert's dense launches on 64-token tiles have d_ff_shared / 128 (gate/up) and d / 256
   // (down) blocks per 64 tokens: split over K until the chip is filled (C4 shape, T = 16: 128 -> 25 us)
   l.ks_sh_gu = l.ks_sh_dn = 1;
-  const bool f32_sh = w->d_ff_shared > 0 && f32_stacks(w->gate_shared_type, w->down_shared_type);
   if (w->d_ff_shared > 0 && l.mode_shared == kSkinny && f32_sh) {
     l.ks_sh_dn = gemm_f32_ksplit((T + 63) / 64, w->d, w->d_ff_shared);
   } else if (w->d_ff_shared > 0 && l.mode_shared == kSkinny) {

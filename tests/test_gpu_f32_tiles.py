@@ -34,11 +34,11 @@ def test_f32_tiles(gpu, monkeypatch, d, d_ff, T):
 
 @pytest.mark.parametrize("T", [20, 96])
 def test_f32_tiles_routed_and_shared(gpu, T):
-    """Unforced: segments of any length, a dense shared expert (the GEMV up to 64 rows, tiles beyond)."""
+    """Unforced: segments of any length, a dense shared expert on the tiles too."""
     spec = em.LayerSpec(d=192, d_ff=320, E=8, k=2, wtype=em.F32, seed=T, weight_std=0.1, d_ff_shared=224)
     hl = em.make_host_layer(spec)
     dl = em.DeviceLayer.upload(hl)
-    assert em.path(dl.desc, T) & em.PATH_TILES64
+    assert em.path(dl.desc, T) & em.PATH_TILES64 and em.path(dl.desc, T) & em.PATH_SHARED_MFMA
     x = em.make_input(spec, T)
     assert rel_l2(run_gpu(hl, x), run_oracle(hl, x)) < 1e-6
 

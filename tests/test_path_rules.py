@@ -1,0 +1,36 @@
+"""Which kernels a layer call takes at the ends of the dispatch rules (ember_moe_path; no GPU): shapes at which a rule taken
+from fewer shapes made calls slower than the kernels they took before it. The figures stand beside the rules."""
+import pytest
+
+import ember_moe as em
+from test_gpu_short_tile_batches import _desc
+
+KERNEL = em.PATH_GEMV | em.PATH_TILES64 | em.PATH_TILES256
+
+
+def _kernel(kw, T):
+    return em.path(_desc(kw), T) & KERNEL
+
+
+F32 = dict(wtype=em.F32)
+
+
+@pytest.mark.parametrize("kw,gemv,tiles", [
+    (dict(F32, d=3072, d_ff=4096, E=16, k=4), 10, 12),
+    (dict(F32, d=2048, d_ff=8192, E=16, k=2), 20, 24),
+    (dict(F32, d=1024, d_ff=2816, E=8, k=2), 10, 12),
+    (dict(F32, d=4096, d_ff=14336, E=8, k=2), 7, 8),
+    (dict(F32, d=2048, d_ff=768, E=128, k=8), 20, 32),
+    (dict(F32, d=1024, d_ff=2816, E=1, k=1), 18, 19),
+    # with an F32 shared expert, both or neither
+    (dict(F32, d=1024, d_ff=768, E=16, k=4, d_ff_shared=2048), 18, 19),
+    (dict(F32, d=512, d_ff=1024, E=16, k=2, d_ff_shared=2048), 18, 19),
+    (dict(F32, d=2048, d_ff=1408, E=64, k=6, d_ff_shared=2816), 18, 20),
+    (dict(F32, d=2048, d_ff=768, E=128, k=2, d_ff_shared=1024), 64, 128),
+])
+def test_f32_gemv_and_tiles(kw, gemv, tiles):
+    assert _kernel(kw, gemv) == em.PATH_GEMV
+    assert _kernel(kw, tiles) == em.PATH_TILES64
+    if "d_ff_shared" in kw:
+        assert not em.path(_desc(kw), gemv) & em.PATH_SHARED_MFMA
+        assert em.path(_desc(kw), tiles) & em.PATH_SHARED_MFMA
