@@ -108,9 +108,13 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, int T, int k, int 
   // 196, T = 300 (28) 213 / 183; F16 T = 256 188 / 190, T = 300 215 / 180; Qwen-shaped T = 512 (32) 350 / 346, T = 1500 528
   // / 456); up to 250 where the 256-token gate/up launch would not give every CU a block (d_ff 2816, E 8, F16: T = 400
   // (100) 99 / 126, T = 768 (192) 134 / 153, T = 1500 (375) 212 / 180)
-  const double most64 = E * ((K_out + 127) / 128) < 256 ? 250.0 : E >= 32 ? 28.0 : 60.0;
-  if (half && (packed || type_in == EMBER_TYPE_F16 || type_out == EMBER_TYPE_F16) && E > 1)
-    return avg_m <= most64 ? kSkinny : kGemm;
+  // A routed layer of one expert, whose launches have the chip to themselves: while the 256-token gate/up launch would
+  // not give every CU a block (64- / 256-token tiles, d 1024, d_ff 2816 F16 T = 900 90 / 122, T = 2048 135 / 143, BF16 T
+  // = 1024 97 / 148; d 4096, d_ff 14336 F16 T = 256 363 / 520, T = 512 472 / 518, T = 700 586 / 574, BF16 T = 800 741 / 666).
+  const int nt = (K_out + 127) / 128;
+  const double most64 = E * nt < 256 ? 250.0 : E >= 32 ? 28.0 : 60.0;
+  if (half && (packed || type_in == EMBER_TYPE_F16 || type_out == EMBER_TYPE_F16) && !dense)
+    return (E == 1 ? std::ceil(avg_m / 256.0) * nt < 256.0 : avg_m <= most64) ? kSkinny : kGemm;
   if (avg_m <= (E > 1 ? 96.0 : half ? 800.0 : q8 ? 1600.0 : 1024.0)) return kSkinny;
   if (type_in == EMBER_TYPE_BF16 && type_out == EMBER_TYPE_BF16 && !packed) return kSkinny;
   return kGemm;

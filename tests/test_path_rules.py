@@ -34,3 +34,19 @@ def test_f32_gemv_and_tiles(kw, gemv, tiles):
     if "d_ff_shared" in kw:
         assert not em.path(_desc(kw), gemv) & em.PATH_SHARED_MFMA
         assert em.path(_desc(kw), tiles) & em.PATH_SHARED_MFMA
+
+
+@pytest.mark.parametrize("wtype", [em.F16, em.BF16])
+def test_one_half_expert_and_shared_lines(wtype):
+    """A routed layer of one expert by its own blocks, not by the 800 rows of a shared expert beside routed launches."""
+    def layer(pack=True, **kw):
+        L = _desc(dict(kw, wtype=wtype))
+        L.prefill_pack = 1 << 20 if pack and wtype == em.BF16 else None
+        return L
+
+    small, big = layer(d=1024, d_ff=2816, E=1, k=1), layer(d=4096, d_ff=14336, E=1, k=1)
+    assert all(em.path(small, T) & KERNEL == em.PATH_TILES64 for T in (200, 801, 1024, 2816))
+    assert em.path(small, 2817) & KERNEL == em.PATH_TILES256
+    assert em.path(big, 512) & KERNEL == em.PATH_TILES64 and em.path(big, 513) & KERNEL == em.PATH_TILES256
+    if wtype == em.BF16:  # without row exponents only the 64-token tiles have the split path
+        assert em.path(layer(False, d=4096, d_ff=14336, E=1, k=1), 4000) & KERNEL == em.PATH_TILES64
