@@ -27,7 +27,8 @@ constexpr int kMaxK = 64;   // picks live in a 64-entry LDS array per wave
 // GEMV, then the FP32 MFMA tiles (64 tokens) at any size.
 enum PathMode { kGemv = 0, kSkinny = 1, kGemm = 2 };
 bool f32_stacks(int type_in, int type_out) { return type_in == EMBER_TYPE_F32 && type_out == EMBER_TYPE_F32; }
-// (K_in = d, K_out = d_ff; with_shared: a shared expert, for F32 stacks one of F32 too; dense: the shared expert, E = 1)
+// (K_in = d, K_out = d_ff; with_shared: a shared expert, for F32 stacks one of F32 too; dense: the shared expert, E = 1; packed: the
+// stacks' own prefill pack, for a Q8_0 shared expert the routed experts')
 int path_mode(int type_in, int K_in, int type_out, int K_out, int T, int k, int E, bool packed = false,
               bool with_shared = false, bool dense = false) {
   const double avg_m = (double)T * k / E;
@@ -97,11 +98,19 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, int T, int k, int 
   } else if (avg_m <= 2.0) {
     return kGemv;
   }
-  // (one dense matrix, the shared expert: the 64-token tiles, split over K (Q8_0: the down projection), up to 800 rows; DeepSeek-shaped layer,
-  // 64- / 256-token tiles: BF16 T = 700 270 / 293 us, T = 850 353 / 302; F16 T = 850 376 / 379, T = 1000 406 / 403;
-  // Q8_0, whose 256-token tiles kept 22 of the chip's CUs busy for longer than all its routed launches, up to 1600:
-  // T = 12 92 / 120, T = 32 96 / 133, T = 100 105 / 154, T = 200 148 / 191, T = 700 230 / 270, T = 1280 328 / 336, T =
-  // 1536 368 / 401, T = 1800 443 / 405)
+  // (one dense matrix, the shared expert: the 64-token tiles, split over K (Q8_0: the down projection), up to 800 rows
+  // in BF16 and F16; DeepSeek-shaped layer, 64- / 256-token tiles: BF16 T = 700 270 / 293 us, T = 850 353 / 302; F16
+  // T = 850 376 / 379, T = 1000 406 / 403.
+  // Q8_0, whose 256-token tiles are few and run longer than small batches' routed launches: while the 64-token gate/up
+  // launch has at most 310 blocks, past which reading the weights again for every 64 rows costs more (DeepSeek-shaped,
+  // d_ff_shared 2816: T = 32 92 / 113, T = 256 149 / 185, T = 700 218 / 262, T = 800 266 / 276, T = 900 288 / 278, T = 1280
+  // 341 / 311; d 2048, 5632, E 60: T = 256 255 / 303, T = 512 306 / 320, T = 600 355 / 327, T = 1024 420 / 369; d 4096,
+  // 4096, E 32: T = 512 323 / 368, T = 600 354 / 346, T = 1280 593 / 467); a narrow one, of fewer than 16 column tiles,
+  // up to 256 rows (DeepSeek-shaped, 1408: T = 256 246 / 254, T = 400 283 / 261, T = 1024 337 / 326); up to 1600 where
+  // the 256-token down launch is few column tiles over a K that outlasts all else (d 1024, 8192, E 32: T = 512 156 / 273,
+  // T = 1024 229 / 305, T = 1536 323 / 351). Beside packed routed tiles, which leave more of the chip, up to 560
+  // blocks, or 400 for d > 2048 (d 2048, 5632, E 60: T = 512 275 / 338, T = 700 314 / 334, T = 900 362 / 344; DeepSeek-
+  // shaped T = 1280 317 / 326, T = 1536 359 / 385; d 4096, 4096, E 32: T = 700 367 / 376, T = 900 405 / 386))
   // BF16 (packed) and F16 routed experts: the 64-token tiles stream the weights best while most experts fit one,
   // up to 60 rows per expert (Mixtral-shaped BF16 T = 160 (40) 589 / 733, T = 256 (64) 789 / 784, T = 384 976 / 848)
   // and, with 32 experts and more, whose counts spread further, up to 28 (DeepSeek-shaped BF16 T = 256 (24) 182 /
@@ -115,7 +124,11 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, int T, int k, int 
   const double most64 = E * nt < 256 ? 250.0 : E >= 32 ? 28.0 : 60.0;
   if (half && (packed || type_in == EMBER_TYPE_F16 || type_out == EMBER_TYPE_F16) && !dense)
     return (E == 1 ? std::ceil(avg_m / 256.0) * nt < 256.0 : avg_m <= most64) ? kSkinny : kGemm;
-  if (avg_m <= (E > 1 ? 96.0 : half ? 800.0 : q8 ? 1600.0 : 1024.0)) return kSkinny;
+  if (q8) {  // (dense)
+    const bool long_down = K_out / ((K_in + 255) / 256) > 1024;
+    return (long_down ? T <= 1600 : nt < 16 ? T <= 256 : (T + 63) / 64 * nt <= (!packed ? 310 : K_in <= 2048 ? 560 : 400)) ? kSkinny : kGemm;
+  }
+  if (avg_m <= (E > 1 ? 96.0 : half ? 800.0 : 1024.0)) return kSkinny;
   if (type_in == EMBER_TYPE_BF16 && type_out == EMBER_TYPE_BF16 && !packed) return kSkinny;
   return kGemm;
 }
@@ -284,7 +297,8 @@ Layout layout_of(const ember_moe_layer* w, int T, bool tight) {
                      f32_stacks(w->gate_type, w->down_type) ? f32_sh : w->d_ff_shared > 0);
   const bool pack_bf16 = w->prefill_pack && bf16_stacks(w);  // row exponents, also the shared expert's if BF16
   l.mode_shared = w->d_ff_shared > 0 ? path_mode(w->gate_shared_type, w->d, w->down_shared_type, w->d_ff_shared,
-                                                 T, 1, 1, pack_bf16 && bf16_shared(w), false, true)
+                                                 T, 1, 1, w->prefill_pack && (q8_shared(w) || (pack_bf16 && bf16_shared(w))),
+                                                 false, true)
                                      : kGemv;
   // a shared expert of the routed experts' types rides in the routed decode launches as one more segment
   // (a few µs), while on its own its T rows make a dense MFMA launch of only d_ff_shared / 128 blocks
@@ -343,8 +357,7 @@ Layout layout_of(const ember_moe_layer* w, int T, bool tight) {
   if (l.ks_sh_dn > 1 && (f32_sh || q8_shared(w))) {
     const size_t y_room = (kMaxKSplit - l.ksplit) * y_part - (tight ? table : 0);
     const size_t h_room = mfma ? slots * w->d_ff * 4 - std::min(align_up(table), slots * w->d_ff * 4) : 0;
-    const size_t fit = std::max(y_room, h_room) / ys_part;
-    while (l.ks_sh_dn > 1 && (size_t)l.ks_sh_dn > fit) l.ks_sh_dn /= 2;
+    l.ks_sh_dn = (int)std::max<size_t>(1, std::min<size_t>(l.ks_sh_dn, std::max(y_room, h_room) / ys_part));
     if (l.ks_sh_dn > 1) l.ys = y_room >= h_room ? l.y + l.ksplit * y_part : l.h + align_up(table);
   }
   // the routed gate/up's tail split (256-token tiles): raw partial gate / up dots [parts][T k][2 d_ff]

@@ -50,3 +50,42 @@ def test_one_half_expert_and_shared_lines(wtype):
     assert em.path(big, 512) & KERNEL == em.PATH_TILES64 and em.path(big, 513) & KERNEL == em.PATH_TILES256
     if wtype == em.BF16:  # without row exponents only the 64-token tiles have the split path
         assert em.path(layer(False, d=4096, d_ff=14336, E=1, k=1), 4000) & KERNEL == em.PATH_TILES64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kw,rows,packed", [
+    (dict(d=1792, d_ff=64, E=2, k=1, d_ff_shared=6400), 384, 704),     # 50 column tiles: 310 and 560 blocks
+    (dict(d=256, d_ff=64, E=2, k=1, d_ff_shared=12288), 1600, 1600),   # one column tile of the down launch
+])
+def test_q8_shared_expert_line(gpu, monkeypatch, kw, rows, packed):
+    """The largest batch whose Q8_0 shared expert takes the 64-token tiles: there the call has the bits of those forced,
+    one row further the 256-token tiles' (the two differ: at these sizes the first split the down projection over
+    K). Held to the FP16 tiles' 2e-3 against the oracle."""
+    import numpy as np
+    import torch
+
+    from gpu_util import rel_l2, run_oracle, same_bits
+
+    hl = em.make_host_layer(em.LayerSpec(seed=6, wtype=em.Q8_0, **kw))
+    dl = em.DeviceLayer.upload(hl)
+    pack = torch.empty(em.prefill_pack_bytes(dl.desc), dtype=torch.uint8, device="cuda")
+    em.prefill_pack(dl.desc, pack)
+
+    def run(x, path=None):
+        monkeypatch.delenv("EMBER_MOE_SHARED_PATH", raising=False)
+        if path:
+            monkeypatch.setenv("EMBER_MOE_SHARED_PATH", path)
+        out, _ = dl.forward(torch.from_numpy(np.ascontiguousarray(x)).cuda())
+        torch.cuda.synchronize()
+        return out.cpu().numpy()
+
+    for p, most in ((None, rows), (pack.data_ptr(), packed)):
+        dl.desc.prefill_pack = p
+        for T in (most, most + 1):
+            x = em.make_input(hl.spec, T)
+            print(f"q8 shared line {kw} T={T} pack={p is not None}", flush=True)
+            y, y64, y256 = run(x), run(x, "skinny"), run(x, "gemm")
+            assert not same_bits(y64, y256)
+            assert same_bits(y, y64 if T == most else y256)
+            if T == rows:
+                assert rel_l2(y, run_oracle(hl, x)) < 2e-3
