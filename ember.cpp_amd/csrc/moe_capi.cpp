@@ -550,7 +550,9 @@ int run_ffn(const ember_moe_layer* w, const float* x, int T, float* out, void* s
     ds.tiles = at<int4>(scratch, l.tiles);
     ds.n_tiles = at<int32_t>(scratch, l.n_tiles);
     ds.tile_bm = gemm_tile_rows(l.mode == kSkinny || l.short_tiles);
-    if (l.mode == kGemm && !l.short_tiles && T > ds.tile_bm) {  // (fewer tokens: one tile per expert, all alike)
+    // (fewer tokens: one tile per expert, all alike)
+    const bool runs = gemm_xcd_runs(w->gate_type, w->prefill_pack) || gemm_xcd_runs(w->down_type, w->prefill_pack);
+    if (l.mode == kGemm && !l.short_tiles && runs && T > ds.tile_bm) {
       ds.xcd = at<int32_t>(scratch, l.n_tiles + 64);
       ds.xcd_tiles = (l.mtiles + 7) / 8;
     }

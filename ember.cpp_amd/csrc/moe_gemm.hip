@@ -271,7 +271,7 @@ __device__ inline int launch_mtiles(const GemmArgs& g, int bm) {
 // XCD-balanced work item of block b for the 256-token-tile kernels: the W = M x NT x KS work items (m-tile
 // major, then n-tile, then K part) are cut into 8 runs, one per XCD (the hardware hands block b to XCD b % 8), and
 // XCD x's j-th block takes item j of run x. The blocks an XCD holds at once mostly share one m-tile of
-// activations in its L2. The runs are of equal time where the dispatch estimated it (GemmArgs::xcd), else of
+// activations in its L2. The runs are of equal time where the dispatch estimated it (GemmArgs::xcd, write_tiles), else of
 // equal length: of Mixtral's ~20 m-tiles at T = 2048 four hold a few rows each, and runs of equal length left
 // some XCDs 280 full tiles and others 224 (CUs without a block a quarter of the time). False: no item (the
 // grid is sized for the largest M).
@@ -1548,6 +1548,12 @@ bool dma_path(int type, bool packed) {
   return dma_enabled() && (type == EMBER_TYPE_Q8_0 || (type == EMBER_TYPE_Q4_K && packed));
 }
 
+// The 256-token tile kernels that follow the dispatch's runs (DispatchScratch::xcd): gemm_kernel's tiles take about
+// the same time whatever their rows.
+bool gemm_xcd_runs(int type, bool packed) {
+  return dma_path(type, packed) || type == EMBER_TYPE_BF16 || type == EMBER_TYPE_F16;
+}
+
 bool gemm_supported(int type, int K) {
   return (type == EMBER_TYPE_Q8_0 || type == EMBER_TYPE_Q4_K || type == EMBER_TYPE_BF16 || type == EMBER_TYPE_F16) &&
          K % GBK == 0;
@@ -1644,7 +1650,7 @@ int launch_gemm_fmt(const GemmArgs& g, int max_mtiles, hipStream_t st) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<FMT, GATED>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemmLds) == hipSuccess;
     if (!lds_ok) return EMBER_ERR_LAUNCH;
-    gk.xcd = nullptr;  // (this kernel's tiles take about the same time whatever their rows)
+    gk.xcd = nullptr;  // (gemm_xcd_runs)
     gemm_kernel<FMT, GATED><<<blocks, kGemmThreads, kGemmLds, st>>>(gk, NT);
     return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
   }

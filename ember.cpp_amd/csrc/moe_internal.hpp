@@ -68,7 +68,7 @@ struct DispatchScratch {
   int32_t* n_tiles = nullptr;
   int tile_bm = 0;
   // optional (null: none), with the tiles: the m-tile position, in kXcdUnit-ths of a tile, at which each XCD's run
-  // of the work begins, [9], runs of equal estimated time and at most xcd_tiles m-tiles
+  // of the work begins, [9], runs of equal length or estimated time (write_tiles) and at most xcd_tiles m-tiles
   int32_t* xcd = nullptr;
   int xcd_tiles = 0;
 };
@@ -358,6 +358,7 @@ inline PackLayout pack_layout(int d, int d_ff, int E, int type) {
 int launch_prefill_pack(int type, const void* W0, const void* W1, int64_t expert_stride, int64_t row_bytes, int E,
                         int N, int K, uint8_t* dst, hipStream_t st);
 bool gemm_supported(int type, int K);
+bool gemm_xcd_runs(int type, bool packed);
 int gemm_max_tiles(int T, int k, int E);
 bool gemm_short_tiles(int type, bool packed, int T, int k, int E, int d_ff);
 int launch_gemm(const GemmArgs& g, bool gated, int max_mtiles, hipStream_t st);

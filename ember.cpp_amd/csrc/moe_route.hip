@@ -343,7 +343,7 @@ __global__ void __launch_bounds__(1024) dispatch_scan(int32_t* __restrict__ chun
     offsets[E] = all;
     *n_used = nu;
   }
-  write_tiles(e, E, tot, off, ds, tmp);
+  write_tiles(e, E, tot, off, nu, ds, tmp);
   if (cnt_lds) {
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += blockDim.x) chunk_cnt[i] = cc[i];
@@ -439,7 +439,7 @@ __global__ void __launch_bounds__(kChunk) dispatch_one_block(const int32_t* __re
     offsets[E] = all;
     *n_used = nu;
   }
-  write_tiles(e, E, tot, off, ds, tmp);
+  write_tiles(e, E, tot, off, nu, ds, tmp);
   __syncthreads();
 #pragma unroll
   for (int c = 0; c < kOneBlockChunks; ++c) {
@@ -503,7 +503,7 @@ __global__ void __launch_bounds__(512) route_dispatch_small(const float* __restr
       if (c > 0) ds.used[upos] = q;
     }
     __syncthreads();
-    write_tiles(q, E, c, off, ds, cnt + E);
+    write_tiles(q, E, c, off, nu, ds, cnt + E);
     if (q < E) cnt[q] = off;
     if (q == 0) {
       ds.offsets[E] = all;

@@ -544,9 +544,9 @@ __device__ inline int block_exclusive_scan(int v, int* tmp, int* total) {
 }
 
 // The GEMM tile table (DispatchScratch::tiles) from the per-expert segment sizes, by the block that
-// computed them: thread q holds expert q's count (q < E; other threads 0). Every thread of the block
+// computed them: thread q holds expert q's count (q < E; other threads 0), n_used of them not 0. Every thread of the block
 // calls it (the scan synchronises), after which ds.tiles holds ceil(count / tile_bm) tiles per expert.
-__device__ inline void write_tiles(int q, int E, int cnt, int off, const DispatchScratch& ds, int* tmp) {
+__device__ inline void write_tiles(int q, int E, int cnt, int off, int n_used, const DispatchScratch& ds, int* tmp) {
   if (!ds.tiles) return;  // uniform over the block
   const int nt = q < E ? (cnt + ds.tile_bm - 1) / ds.tile_bm : 0;
   const int h = tile_height(cnt, ds.tile_bm);
@@ -555,16 +555,22 @@ __device__ inline void write_tiles(int q, int E, int cnt, int off, const Dispatc
   for (int i = 0; i < nt; ++i) ds.tiles[base + i] = make_int4(q, off + i * h, min(h, cnt - i * h), 0);
   if (q == 0) *ds.n_tiles = all;
   if (!ds.xcd) return;
-  // Where the tiles' work reaches each eighth (DispatchScratch::xcd). The rest of a segment past whole tiles
-  // (at most 32 rows, tile_height) counts 6/13 of a tile, its measured time in the 256-token DMA kernels, when
-  // such rests are at least a sixth of the tiles (Mixtral-shaped T = 1050, most experts just past 256 rows, 1085 ->
-  // 955 us; T = 2048 1775 -> 1737). Otherwise all tiles count alike: runs of equal length that fill whole
-  // rounds of blocks are worth more (T = 1200, one rest in 16 tiles, 1132 us, weighted 1192; T = 512, weighted by
-  // 32-row steps, 512 -> 589).
+  // Where the tiles' work reaches each eighth (DispatchScratch::xcd). The rest of a segment past whole tiles (at most 32
+  // rows, tile_height) counts 6/13 of a tile, its time in the 256-token DMA kernels, when at least half of the experts
+  // end in such a rest and no other tile has 224 rows or fewer. Otherwise all tiles count alike: runs of equal length fill
+  // whole rounds of blocks, which is worth more than weights that miss some tiles' time. By time / by length, us:
+  // taken, Mixtral-shaped Q8_0 T = 1008 943 / 995, T = 1056 987 / 1013, T = 2048 (4 rests for 8 experts) 1669 / 1712,
+  // BF16 T = 1008 1301 / 1381, d 1024, d_ff 2816, E 8 Q8_0 rows T = 1024 155 / 178; not taken, Mixtral-shaped T = 1120 (7
+  // rests, a pair of 160-row tiles) Q8_0 1064 / 1038, BF16 1651 / 1472, T = 2128 (6 rests, tiles of 192) Q8_0 1841 / 1760,
+  // d 3072, d_ff 4096, E 16 T = 1120 Q4_K 522 / 464, T = 1008 (5 rests for 16 experts) BF16 623 / 557. Of 421 calls of
+  // eight shapes in all encodings 60 are taken: 0.99 to 1.14 times as fast, 1.04 in the mean.
   const int rest = cnt - (nt - 1) * h;
   const bool light = nt > 1 && rest <= 32;
-  const bool weigh = 6 * __syncthreads_count(light) >= all;
-  const int wh = 13 * 64, wl = light && weigh ? 6 * 64 : wh;
+  if (2 * __syncthreads_count(light) < n_used || __syncthreads_or(nt > 0 && min(h, cnt) <= 224)) {
+    if (q < 9) ds.xcd[q] = (int)((int64_t)all * kXcdUnit * q / 8);
+    return;
+  }
+  const int wh = 13 * 64, wl = light ? 6 * 64 : wh;
   const int we = nt > 0 ? (nt - 1) * wh + wl : 0;
   int wall = 0;
   const int wbase = block_exclusive_scan(we, tmp, &wall);

@@ -47,6 +47,82 @@ def test_half_tiles_ragged(gpu, monkeypatch, wtype, pack, shared, T):
     assert same_bits(y, run_gpu(hl, x, pack=pack))
 
 
+def _runs(counts):
+    """write_tiles' rule: tile heights, the XCDs' runs in 4096ths of a tile, and whether they follow the tiles' time."""
+    tiles, weight, light, short = [], [], 0, False
+    for n in counts:
+        nt = -(-n // 256)
+        h = 256 if nt <= 1 or n - (nt - 1) * 256 <= 32 else -(-(-(-n // nt)) // 32) * 32
+        rows = [min(h, n - i * h) for i in range(nt)]
+        rest = nt > 1 and rows[-1] <= 32
+        light, short = light + rest, short or (nt > 0 and min(h, n) <= 224)
+        tiles += rows
+        weight += [832] * (nt - 1) + [384 if rest else 832] if nt else []
+    timed = 2 * light >= sum(n > 0 for n in counts) and not short
+    total, pos = sum(weight), []
+    for x in range(9):
+        if not timed:
+            pos.append(len(tiles) * 4096 * x // 8)
+            continue
+        r, i = total * x // 8, 0
+        while i < len(weight) - 1 and r >= weight[i]:
+            r, i = r - weight[i], i + 1
+        pos.append(i * 4096 + min(r * 4096 // weight[i], 4096))
+    return tiles, pos, timed
+
+
+def _routed_to(counts, d, seed):
+    """Tokens that a one-hot router sends to expert e counts[e] times, in a shuffled order."""
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((sum(counts), d)).astype(np.float32) * 0.5
+    e = rng.permutation(np.repeat(np.arange(len(counts)), counts))
+    x[:, :len(counts)] = 0.0
+    x[np.arange(len(e)), e] = 8.0
+    return x
+
+
+@pytest.mark.parametrize("counts,timed", [
+    ((270, 262, 256, 250), True),           # two rests for four experts
+    ((530, 514, 512, 500, 0, 257), True),   # rests behind two whole tiles, an expert without rows
+    ((288, 288, 288, 288), True),
+    ((270, 256, 256, 250), False),          # one rest
+    ((270, 262, 289, 270), False),          # a pair of 160-row tiles
+    ((270, 262, 150, 270), False),          # a tile of 150 rows
+    ((700, 33, 0, 290), False),             # three tiles of 256, 256, 188; pairs
+])
+@pytest.mark.parametrize("wtype,pack", [(em.Q8_0, True), (em.Q4_K, True), (em.Q8_0, False), (em.BF16, True), (em.F16, False)])
+def test_xcd_runs(gpu, monkeypatch, wtype, pack, counts, timed):
+    """The tiles' number and the runs that the dispatch leaves in the scratch (the count in its last 256 bytes, the runs 64
+    bytes on), by the rule restated above, and the output of segments of just these lengths against the oracle."""
+    import torch
+
+    monkeypatch.setenv("EMBER_MOE_PATH", "gemm")
+    monkeypatch.setenv("EMBER_GEMM_SHORT", "0")  # 256-row tiles whatever the rule for 64-row ones says
+    monkeypatch.setenv("EMBER_TAIL_PARTS", "1")
+    E = len(counts)
+    spec = em.LayerSpec(d=256, d_ff=512, E=E, k=1, wtype=wtype, seed=9)
+    hl = em.make_host_layer(spec)
+    hl.router = np.ascontiguousarray(np.eye(E, 256, dtype=np.float32).reshape(-1))
+    x = _routed_to(counts, 256, 9)
+    T = len(x)
+    dl = em.DeviceLayer.upload(hl)
+    if pack:
+        buf = torch.empty(em.prefill_pack_bytes(dl.desc), dtype=torch.uint8, device="cuda")
+        em.prefill_pack(dl.desc, buf)
+        dl.tensors["pack"] = buf
+    print(f"xcd runs {em.TYPE_NAMES[wtype]} pack={pack} {counts}", flush=True)
+    y, scratch = dl.forward(torch.from_numpy(x).cuda())
+    torch.cuda.synchronize()
+    assert em.path(dl.desc, T) & em.PATH_TILES256
+    offsets = em.scratch_routing(dl.desc, T, scratch)["offsets"]
+    assert np.array_equal(np.diff(offsets), counts)
+    tail = scratch[em.scratch_bytes(dl.desc, T) - 256:][:100].cpu().numpy().view(np.int32)
+    tiles, pos, by_time = _runs(counts)
+    assert by_time == timed and tail[0] == len(tiles)
+    assert list(tail[16:25]) == pos
+    assert rel_l2(y.cpu().numpy(), run_oracle(hl, x)) < 2e-3
+
+
 @pytest.mark.parametrize("T", [1050, 2048])
 def test_xcd_runs_skewed(gpu, T):
     """Uniform and skewed segments of eight experts: full tiles, equal tiles and light rests mixed."""
