@@ -896,8 +896,7 @@ __global__ void __launch_bounds__(kDmaThreads, (2 * DmaRing<WF, SHORT>::kBlocks)
 }
 
 // The 256-token DMA kernel for BF16 (with the row exponents of a prefill pack) and F16 rows: gemm_dma_q8_kernel's
-// layout (2 (M) x 4 (N) waves of 128 x 64, subtiles past the tile's rows skipped, XCD runs, K split of the plain
-// projection) with K tiles of 32 columns, so that both operands of a stage (16 KiB each) fit a ring of four,
+// layout (2 (M) x 4 (N) waves of 128 x 64, subtiles past the tile's rows skipped, XCD runs; no K split) with K tiles of 32 columns, so that both operands of a stage (16 KiB each) fit a ring of four,
 // three tiles in flight. A tile row is 64 bytes, four granules, XOR-swizzled so that the 16 rows one read pass
 // touches fall on distinct banks. A B fragment is one 16-byte read; BF16 values are scaled by the row's power of two
 // and rounded to fp16 on the way to the MFMA, as the register-staged kernel does, whose outputs these equal
@@ -913,15 +912,12 @@ template <int FMT, bool GATED>
 __global__ void __launch_bounds__(kDmaThreads) gemm_dma_half_kernel(GemmArgs g, int NT) {
   constexpr int BN = GATED ? 128 : 256, NS = kHalfStages;
   extern __shared__ __align__(16) uint8_t dsm[];
-  const int KS = GATED ? 1 : g.ksplit;
-  int mt, rem, e, p0, rows;
-  if (!xcd_item(g, launch_mtiles(g, GBM), NT, KS, mt, rem)) return;
-  const int nt = rem / KS, ks = rem % KS;
+  int mt, nt, e, p0, rows;
+  if (!xcd_item(g, launch_mtiles(g, GBM), NT, 1, mt, nt)) return;
   row_tile(g, mt, GBM, e, p0, rows);
   if (rows <= 0) return;
   const int n0 = nt * BN, K = g.K, N = g.N;
-  const int nk_all = K / kHalfBK;
-  const int kt0 = ks * nk_all / KS, nk = (ks + 1) * nk_all / KS - kt0;
+  const int nk = K / kHalfBK;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 2, wn = wave & 3;
@@ -942,7 +938,7 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_half_kernel(GemmArgs g, 
   // tile kt (clamped: tiles past the end reload the last, never multiplied) into the stage at byte `st`.
   // NOA: this wave's activation rows (32 w .. 32 w + 31) lie past the tile's tokens, so it loads none.
   auto issue = [&](int kt, int st, auto NOAc) {
-    const size_t o = (size_t)(kt0 + min(kt, nk - 1)) * kHalfBK * 2;
+    const size_t o = (size_t)min(kt, nk - 1) * kHalfBK * 2;
 #pragma unroll
     for (int i = 0; i < kHalfInst; ++i) {
       if constexpr (!decltype(NOAc)::value) lds_dma16(srcA[i] + o, dsm + st + 1024 * (kHalfInst * wave + i));
@@ -1091,7 +1087,7 @@ __global__ void __launch_bounds__(kDmaThreads) gemm_dma_half_kernel(GemmArgs g, 
             store_h(g, o, p0 + m, ex, __builtin_ldexpf(acc[i][0][4 * ii + jj], we0),
                     __builtin_ldexpf(acc[i][1][4 * ii + jj], we1), n == n0, weh);
           } else {
-            g.out_y[ks * g.part_stride + o] = unscale_y(__builtin_ldexpf(acc[i][jn][4 * ii + jj], we0), ex);
+            g.out_y[o] = unscale_y(__builtin_ldexpf(acc[i][jn][4 * ii + jj], we0), ex);
           }
         }
     }
@@ -1618,8 +1614,7 @@ int launch_gemm_fmt(const GemmArgs& g, int max_mtiles, hipStream_t st) {
         hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_dma_half_kernel<FMT, GATED>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kHalfLds) == hipSuccess;
     if (!ok) return EMBER_ERR_LAUNCH;
-    if (GATED || gk.ksplit < 1) gk.ksplit = 1;
-    gemm_dma_half_kernel<FMT, GATED><<<blocks * (unsigned)gk.ksplit, kDmaThreads, kHalfLds, st>>>(gk, NT);
+    gemm_dma_half_kernel<FMT, GATED><<<blocks, kDmaThreads, kHalfLds, st>>>(gk, NT);
     return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
   } else if (dma_path(FMT, g.Wp != nullptr)) {
     if (GATED || gk.ksplit < 1) gk.ksplit = 1;
@@ -1777,7 +1772,7 @@ bool gemm_short_tiles(int type, bool packed, int T, int k, int E, int d_ff) {
 int gemm_expected_tiles(int T, int k, int E) { return (int)std::ceil(expected_row_tiles(T, k, E, SBM)); }
 
 int gemm_ksplit(int type, bool packed, int T, int k, int E, int N, int K) {
-  if (!dma_path(type, packed)) return 1;  // the split lives in the DMA kernels
+  if (!dma_path(type, packed)) return 1;  // gemm_dma_q8_kernel alone splits K
   // tuning override, clamped so that every part holds at least one K tile
   if (const char* v = std::getenv("EMBER_KSPLIT")) return std::max(1, std::min(std::min(kMaxKSplit, K / GBK), atoi(v)));
   // The launch runs tiles * ks blocks in rounds of `slots`; a part of a round costs a whole round, so ks

@@ -2,7 +2,7 @@
 one tile, the rest of at most 32 rows past whole tiles (left as it is and, being more than a sixth of the tiles,
 counted as light), and equal tiles in 32-row steps. A row's sums do not depend on its tile, so every
 row's bits are those of the same token in a call of at most 256 tokens (one tile per expert), and the output holds
-the oracle's bar (utils.cpp:704-748), with the down projection split over K or not."""
+the oracle's bar (utils.cpp:704-748), with the down projection split over K (Q8_0, Q4_K) or not."""
 import numpy as np
 import pytest
 
@@ -25,16 +25,17 @@ def test_tile_heights(gpu, monkeypatch, wtype, pack, E, T):
     assert rel_l2(y, run_oracle(hl, x)) < 2e-3
     for a in range(0, T, 200):
         assert same_bits(y[a:a + 200], run_gpu(hl, x[a:a + 200], pack=pack)), a
-    monkeypatch.setenv("EMBER_KSPLIT", "4")
-    assert rel_l2(run_gpu(hl, x, pack=pack), y) < 1e-5
+    if wtype not in (em.BF16, em.F16):  # (whose 256-token tiles do not split K)
+        monkeypatch.setenv("EMBER_KSPLIT", "4")
+        assert rel_l2(run_gpu(hl, x, pack=pack), y) < 1e-5
 
 
 @pytest.mark.parametrize("T", [31, 32, 33, 96, 97, 129, 256, 300])
 @pytest.mark.parametrize("wtype,pack,shared", [(em.BF16, True, 0), (em.F16, False, 0), (em.BF16, True, 192)])
 def test_half_tiles_ragged(gpu, monkeypatch, wtype, pack, shared, T):
     """The BF16 / F16 256-token tiles: subtiles and activation loads past a tile's rows left out, weight rows past
-    d_ff and d (320 = 2.5 x 128, 192 < 256), an even and an odd number of 32-column K tiles per part, a dense shared
-    expert, against the oracle at the fp16 operands' 2e-3."""
+    d_ff and d (320 = 2.5 x 128, 192 < 256), 6 and 10 K tiles of 32 columns (no multiple of the
+    ring's four stages), a dense shared expert, against the oracle at the fp16 operands' 2e-3."""
     spec = em.LayerSpec(d=192, d_ff=320, E=3, k=3, wtype=wtype, seed=T, d_ff_shared=shared)
     hl = em.make_host_layer(spec)
     x = em.make_input(spec, T)
