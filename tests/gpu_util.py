@@ -12,9 +12,9 @@ def rel_l2(a, b) -> float:
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30))
 
 
-def run_gpu(hl: em.HostLayer, x: np.ndarray, pack: bool = False):
+def run_gpu(hl: em.HostLayer, x: np.ndarray, pack: bool = False, whole: bool = False):
     """Uploads the layer and x (pack: with the layer's prefill pack), runs ember_moe_ffn, returns out as
-    numpy."""
+    numpy (whole: with the scratch and the device layer)."""
     import torch
 
     dl = em.DeviceLayer.upload(hl)
@@ -23,9 +23,16 @@ def run_gpu(hl: em.HostLayer, x: np.ndarray, pack: bool = False):
         em.prefill_pack(dl.desc, buf)
         dl.tensors["pack"] = buf
     xd = torch.from_numpy(np.ascontiguousarray(x, np.float32)).cuda()
-    out, _ = dl.forward(xd)
+    out, scratch = dl.forward(xd)
     torch.cuda.synchronize()
-    return out.cpu().numpy()
+    return (out.cpu().numpy(), scratch, dl) if whole else out.cpu().numpy()
+
+
+def tile_table_tail(desc, T: int, scratch):
+    """What the dispatch of a call on the tiles left in the last 256 bytes of its scratch: the number of row tiles, and 64
+    bytes on the XCDs' runs [9] (of 256-row tiles)."""
+    tail = scratch[em.scratch_bytes(desc, T) - 256:][:100].cpu().numpy().view(np.int32)
+    return int(tail[0]), list(tail[16:25])
 
 
 def run_oracle(hl: em.HostLayer, x: np.ndarray, nthreads: int = 0):

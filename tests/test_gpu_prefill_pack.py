@@ -30,10 +30,13 @@ def _run(hl, x, pack: bool):
 
 
 # more than 1.5 tokens per expert: the 256-token-tile GEMM (short segments skip their empty subtiles);
-# d_ff 704 and d 576 leave partial n-tiles
+# d_ff 704 and d 576 leave partial n-tiles; short "0": the packs on 256-row tiles, not the 64-row ones that their
+# rules choose for most of these
+@pytest.mark.parametrize("short", ["1", "0"])
 @pytest.mark.parametrize("d,d_ff,E,k,T", [(512, 1024, 4, 2, 320), (576, 704, 4, 2, 300), (256, 512, 8, 2, 1024),
                                           (512, 1024, 4, 2, 64), (576, 704, 4, 2, 37), (256, 512, 8, 2, 150)])
-def test_pack_same_bits_as_rows(gpu, d, d_ff, E, k, T):
+def test_pack_same_bits_as_rows(gpu, monkeypatch, d, d_ff, E, k, T, short):
+    monkeypatch.setenv("EMBER_GEMM_SHORT", short)
     spec = em.LayerSpec(d=d, d_ff=d_ff, E=E, k=k, wtype=em.Q8_0, seed=21)
     hl = em.make_host_layer(spec)
     x = em.make_input(spec, T)
@@ -58,9 +61,10 @@ def test_pack_deepseek_style_with_shared_expert(gpu):
 
 
 # Q4_K: d, d_ff multiples of 256; more than 2 tokens per expert takes the 256-token tiles
+@pytest.mark.parametrize("short", ["1", "0"])
 @pytest.mark.parametrize("d,d_ff,E,k,T", [(512, 768, 8, 2, 320), (256, 512, 4, 2, 1000), (768, 512, 16, 4, 700),
                                           (512, 768, 8, 2, 40)])
-def test_q4_k_pack_same_bits_as_register_staged(gpu, monkeypatch, d, d_ff, E, k, T):
+def test_q4_k_pack_same_bits_as_register_staged(gpu, monkeypatch, d, d_ff, E, k, T, short):
     """Both runs forced onto the 256-token tiles (EMBER_MOE_PATH=gemm): the packed DMA kernel and the
     register-staged one form the same fp16 operands and pair the same K elements in each MFMA. (The DMA
     kernel's tail split, which sums the K parts of the last round's tiles separately, is off for the
@@ -68,7 +72,8 @@ def test_q4_k_pack_same_bits_as_register_staged(gpu, monkeypatch, d, d_ff, E, k,
     spec = em.LayerSpec(d=d, d_ff=d_ff, E=E, k=k, wtype=em.Q4_K, seed=24)
     hl = em.make_host_layer(spec)
     x = em.make_input(spec, T)
-    print(f"prefill pack q4_k d={d} d_ff={d_ff} E={E} T={T}", flush=True)
+    print(f"prefill pack q4_k d={d} d_ff={d_ff} E={E} T={T} short={short}", flush=True)
+    monkeypatch.setenv("EMBER_GEMM_SHORT", short)
     y_default = _run(hl, x, pack=True)
     monkeypatch.setenv("EMBER_MOE_PATH", "gemm")
     monkeypatch.setenv("EMBER_TAIL_PARTS", "1")
@@ -80,13 +85,15 @@ def test_q4_k_pack_same_bits_as_register_staged(gpu, monkeypatch, d, d_ff, E, k,
     assert rel_l2(y_default, run_oracle(hl, x)) < 2e-3
 
 
-def test_q4_k_pack_with_k_split(gpu):
+@pytest.mark.parametrize("short", ["1", "0"])
+def test_q4_k_pack_with_k_split(gpu, monkeypatch, short):
     """A long down projection (d_ff 4096) on few blocks: the DMA kernel splits its K and the combine adds
     the parts in a fixed order, so the bits differ from the unsplit kernel's but the oracle's bar holds."""
     spec = em.LayerSpec(d=256, d_ff=4096, E=4, k=2, wtype=em.Q4_K, seed=25)
     hl = em.make_host_layer(spec)
     x = em.make_input(spec, 512)
-    print("prefill pack q4_k K split", flush=True)
+    print(f"prefill pack q4_k K split short={short}", flush=True)
+    monkeypatch.setenv("EMBER_GEMM_SHORT", short)
     y_pack = _run(hl, x, pack=True)
     assert rel_l2(y_pack, _run(hl, x, pack=False)) < 1e-5
     assert rel_l2(y_pack, run_oracle(hl, x)) < 2e-3

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 import ember_moe as em
-from gpu_util import rel_l2, run_oracle, same_bits
+from gpu_util import rel_l2, run_oracle, same_bits, tile_table_tail
 
 
 def _layer(kw, pack=True):
@@ -32,11 +32,13 @@ def _run(dl, x):
     return out.cpu().numpy()
 
 
-WIDE = dict(d=512, d_ff=512, E=64, k=2)  # 64 experts x 4 column tiles: a block for every CU
-FEW = dict(d=512, d_ff=768, E=4, k=2)
+# (a selection bias of the scores' own spread skews the segments, so that some pass 64 rows)
+WIDE = dict(d=512, d_ff=512, E=64, k=2, bias_std=0.02)  # 64 experts x 4 column tiles: a block for every CU
+FEW = dict(d=512, d_ff=768, E=4, k=2, bias_std=0.15)
 CASES = {
-    # name: (spec kwargs, T): T k / E mean rows, the rule's ends and segments past 64 rows
-    "q8_first": (dict(WIDE, wtype=em.Q8_0), 65),
+    # name: (spec kwargs, T): T k / E mean rows, the rule's ends and segments past 64 rows ("past" and "below": the batch
+    # next to an end that keeps 256-row tiles)
+    "q8_first": (dict(WIDE, wtype=em.Q8_0, bias_std=0.3), 65),
     "q8_last": (dict(WIDE, wtype=em.Q8_0), 1280),
     "q8_past": (dict(WIDE, wtype=em.Q8_0), 1281),
     "q4_last": (dict(WIDE, wtype=em.Q4_K), 1856),
@@ -57,9 +59,18 @@ def test_short_tiles_of_batches_same_bits(gpu, monkeypatch, name):
     monkeypatch.setenv("EMBER_MOE_PATH", "gemm")
     monkeypatch.setenv("EMBER_TAIL_PARTS", "1")
     print(f"short tiles of a batch {name} T={T}", flush=True)
-    y = _run(dl, x)
-    monkeypatch.setenv("EMBER_GEMM_SHORT", "0")
-    assert same_bits(y, _run(dl, x))
+    import torch
+
+    out, scratch = dl.forward(torch.from_numpy(np.ascontiguousarray(x)).cuda())
+    torch.cuda.synchronize()
+    y = out.cpu().numpy()
+    counts = np.diff(em.scratch_routing(dl.desc, T, scratch)["offsets"])
+    rows = 256 if name.endswith(("past", "below")) else 64
+    assert tile_table_tail(dl.desc, T, scratch)[0] == int(np.sum(-(-counts // rows)))
+    assert np.sum(-(-counts // 64)) > np.sum(-(-counts // 256))
+    if rows == 64:
+        monkeypatch.setenv("EMBER_GEMM_SHORT", "0")
+        assert same_bits(y, _run(dl, x))
     err = rel_l2(y, run_oracle(hl, x))
     print(f"  rel-L2 vs oracle {err:.2e}", flush=True)
     assert err < 2e-3, err

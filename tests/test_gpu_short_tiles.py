@@ -1,6 +1,6 @@
 """The 256-token DMA tile kernels' short variant: a launch of at most 64 tokens has no segment, hence no tile,
-of more than 64 rows (a token picks an expert once), so its LDS stages hold 64 activation rows and five
-stages fit (four tiles in flight instead of two). It multiplies the same fragments in the same order as the
+of more than 64 rows (a token picks an expert once), so its LDS stages hold 64 activation rows: five stages for ggml
+rows, three (Q8_0) or four (Q4_K) in half a CU's LDS for the packs. It multiplies the same fragments in the same order as the
 three-stage kernel, so its outputs are bit-identical to it (EMBER_GEMM_SHORT=0 forces the three-stage
 kernel), and held to the oracle (utils.cpp:704-748) at the 2e-3 rel-L2 bar; 65 tokens take the three-stage
 kernel."""

@@ -32,8 +32,9 @@ CASES = {
 }
 
 
+@pytest.mark.parametrize("short", ["1", "0"])  # the 64-row ring that launches this small take, the 256-row one
 @pytest.mark.parametrize("name", sorted(CASES))
-def test_tail_split(gpu, monkeypatch, name):
+def test_tail_split(gpu, monkeypatch, name, short):
     import torch
 
     kw, T = CASES[name]
@@ -44,6 +45,7 @@ def test_tail_split(gpu, monkeypatch, name):
     em.prefill_pack(dl.desc, buf)
     dl.tensors["pack"] = buf
     x = em.make_input(spec, T, seed=52)
+    monkeypatch.setenv("EMBER_GEMM_SHORT", short)
     monkeypatch.setenv("EMBER_MOE_PATH", "gemm")  # the 256-token tiles
     monkeypatch.setenv("EMBER_TAIL_PARTS", "8")   # the split, also for these short K (by default K >= 64 tiles)
     assert em.path(dl.desc, T) & em.PATH_TILES256

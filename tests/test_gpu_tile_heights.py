@@ -1,13 +1,13 @@
 """The 256-token tiles' heights and the XCDs' runs of work: with k = E every expert holds all T tokens, so T walks
-one tile, the rest of at most 32 rows past whole tiles (left as it is and, being more than a sixth of the tiles,
-counted as light), and equal tiles in 32-row steps. A row's sums do not depend on its tile, so every
-row's bits are those of the same token in a call of at most 256 tokens (one tile per expert), and the output holds
+one tile, the rest of at most 32 rows past whole tiles (left as it is and, every expert ending in one, counted as
+light), and equal tiles in 32-row steps. EMBER_GEMM_SHORT=0 keeps the packs, whose rule for 64-row tiles takes
+layers this small, on 256-row tiles. A row's sums do not depend on its tile, so every row's bits are those of the same token in a call of at most 256 tokens (one tile per expert), and the output holds
 the oracle's bar (utils.cpp:704-748), with the down projection split over K (Q8_0, Q4_K) or not."""
 import numpy as np
 import pytest
 
 import ember_moe as em
-from gpu_util import rel_l2, run_gpu, run_oracle, same_bits
+from gpu_util import rel_l2, run_gpu, run_oracle, same_bits, tile_table_tail
 
 pytestmark = pytest.mark.gpu
 
@@ -19,6 +19,7 @@ def test_tile_heights(gpu, monkeypatch, wtype, pack, E, T):
     hl = em.make_host_layer(spec)
     x = em.make_input(spec, T)
     monkeypatch.setenv("EMBER_MOE_PATH", "gemm")
+    monkeypatch.setenv("EMBER_GEMM_SHORT", "0")
     monkeypatch.setenv("EMBER_KSPLIT", "1")
     print(f"tile heights {em.TYPE_NAMES[wtype]} pack={pack} T={T}", flush=True)
     y = run_gpu(hl, x, pack=pack)
@@ -117,19 +118,21 @@ def test_xcd_runs(gpu, monkeypatch, wtype, pack, counts, timed):
     assert em.path(dl.desc, T) & em.PATH_TILES256
     offsets = em.scratch_routing(dl.desc, T, scratch)["offsets"]
     assert np.array_equal(np.diff(offsets), counts)
-    tail = scratch[em.scratch_bytes(dl.desc, T) - 256:][:100].cpu().numpy().view(np.int32)
     tiles, pos, by_time = _runs(counts)
-    assert by_time == timed and tail[0] == len(tiles)
-    assert list(tail[16:25]) == pos
+    assert by_time == timed
+    assert tile_table_tail(dl.desc, T, scratch) == (len(tiles), pos)
     assert rel_l2(y.cpu().numpy(), run_oracle(hl, x)) < 2e-3
 
 
 @pytest.mark.parametrize("T", [1050, 2048])
-def test_xcd_runs_skewed(gpu, T):
+def test_xcd_runs_skewed(gpu, monkeypatch, T):
     """Uniform and skewed segments of eight experts: full tiles, equal tiles and light rests mixed."""
+    monkeypatch.setenv("EMBER_GEMM_SHORT", "0")
     spec = em.LayerSpec(d=256, d_ff=512, E=8, k=2, wtype=em.Q8_0, seed=9, router_std=0.01 if T == 1050 else 0.2)
     hl = em.make_host_layer(spec)
     x = em.make_input(spec, T)
-    y = run_gpu(hl, x, pack=True)
+    y, scratch, dl = run_gpu(hl, x, pack=True, whole=True)
+    tiles, pos, _ = _runs(np.diff(em.scratch_routing(dl.desc, T, scratch)["offsets"]))
+    assert tile_table_tail(dl.desc, T, scratch) == (len(tiles), pos)
     assert np.isfinite(y).all()
     assert rel_l2(y, run_oracle(hl, x)) < 2e-3
