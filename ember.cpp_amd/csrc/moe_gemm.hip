@@ -1819,9 +1819,6 @@ int launch_act_conv(const ActConv& c, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? EMBER_OK : EMBER_ERR_LAUNCH;
 }
 
-// Tile table for the grouped GEMMs: (expert, first token) of every bm-token tile of every expert
-// segment with tokens, ascending by expert. One thread; E entries of offsets.
-
 int gemm_tile_rows(bool skinny) { return skinny ? SBM : GBM; }
 
 

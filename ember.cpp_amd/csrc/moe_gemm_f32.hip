@@ -17,9 +17,8 @@
 // chains of 64 columns are added up, and those sums are accumulated with Kahan's compensation: no more
 // roundings deep than the GEMV at any K (layer error against 64 bits 1.6e-7 to 1.7e-7, the GEMV's 1.6e-7 to
 // 2.0e-7). The additions are not hidden (FP32 MFMAs and FP32 VALU instructions do not overlap on gfx950: 4 of
-// each take the sum of their times, and the counters put this kernel's MFMA and VALU cycles together at 93 %
-// of its time): 11 of them per 64 columns and output, a third of the MFMA time,
-// and a twelfth instruction that keeps infinite sums infinite.
+// each take the sum of their times; d 1024, d_ff 2816, E 8, 400 tokens, gate/up: MFMAs 47 % of the cycles, vector
+// instructions 28 %): 11 of them per 64 columns and output, and a twelfth that keeps infinite sums infinite.
 #include <cstdlib>
 #include <type_traits>
 

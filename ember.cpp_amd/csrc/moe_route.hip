@@ -648,7 +648,7 @@ __global__ void __launch_bounds__(256) router_logits_chains(const float* __restr
 // NT such tiles side by side in the experts, a pair of waves shares them and their sums meet in LDS. Operands come
 // straight from memory, U steps of 32 elements ahead (the 16 rows of a wave's load are half lines, the pair's other
 // wave takes the other halves). Bound: the FP64 matrix rate, 48 TFLOP/s as measured (105 cycles per MFMA): E = 128,
-// d = 2048, T = 4096 takes 53 us of which 45 at that rate; the FMAs of router_logits_chains, which read both
+// d = 2048, T = 4096 takes 53 to 61 us of which 45 at that rate; the FMAs of router_logits_chains, which read both
 // operands from LDS for every few of them, took 88.
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 template <int NT, int U>
