@@ -18,6 +18,10 @@ CASES = {
                                                                            "EMBER_TAIL_PARTS": "8"}, em.PATH_TILES256),
     "tiles_q4_shared": (dict(d=512, d_ff=768, E=8, k=2, wtype=em.Q4_K, d_ff_shared=512), 24,
                         {"EMBER_MOE_PATH": "gemm"}, em.PATH_TILES256),
+    # the shared expert's down parts, written on the side stream, in y and (y full) in h
+    "tiles_q8_shared_in_y": (dict(d=512, d_ff=512, E=8, k=2, wtype=em.Q8_0, d_ff_shared=1024), 40, {}, em.PATH_SHARED_MFMA),
+    "tiles_q8_shared_in_h": (dict(d=256, d_ff=8192, E=4, k=1, wtype=em.Q8_0, d_ff_shared=1024), 30, {}, em.PATH_SHARED_MFMA),
+    "tiles_f32_shared": (dict(d=512, d_ff=1024, E=16, k=2, wtype=em.F32, d_ff_shared=2048), 100, {}, em.PATH_SHARED_MFMA),
 }
 CALLS = 4  # layer calls per graph (two copies of the layer, alternating)
 
@@ -31,8 +35,9 @@ def test_graph_replays_match_eager(gpu, monkeypatch, name):
         monkeypatch.setenv(k, v)
     spec = em.LayerSpec(seed=81, **kw)
     dl = em.DeviceLayer.upload(em.make_host_layer(spec))
-    dl.tensors["pack"] = torch.empty(em.prefill_pack_bytes(dl.desc), dtype=torch.uint8, device="cuda")
-    em.prefill_pack(dl.desc, dl.tensors["pack"])
+    if em.prefill_pack_bytes(dl.desc):
+        dl.tensors["pack"] = torch.empty(em.prefill_pack_bytes(dl.desc), dtype=torch.uint8, device="cuda")
+        em.prefill_pack(dl.desc, dl.tensors["pack"])
     dls = [dl, dl.clone()]
     assert em.path(dl.desc, T) & bit
     print(f"graph replay {name} T={T}", flush=True)
