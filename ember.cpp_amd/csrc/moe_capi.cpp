@@ -27,8 +27,8 @@ constexpr int kMaxK = 64;   // picks live in a 64-entry LDS array per wave
 // GEMV, then the FP32 MFMA tiles (64 tokens) at any size.
 enum PathMode { kGemv = 0, kSkinny = 1, kGemm = 2 };
 bool f32_stacks(int type_in, int type_out) { return type_in == EMBER_TYPE_F32 && type_out == EMBER_TYPE_F32; }
-// (K_in = d, K_out = d_ff; with_shared: a shared expert, for F32 stacks one of F32 too; dense: the shared expert, E = 1; packed: the
-// stacks' own prefill pack, for a Q8_0 shared expert the routed experts')
+// (K_in = d, K_out = d_ff; packed: the stacks' own prefill pack, for a Q8_0 shared expert the routed experts';
+// with_shared: a shared expert, for F32 stacks one of F32 too; dense: the shared expert, E = 1)
 int path_mode(int type_in, int K_in, int type_out, int K_out, int T, int k, int E, bool packed = false,
               bool with_shared = false, bool dense = false) {
   const double avg_m = (double)T * k / E;
@@ -126,7 +126,8 @@ int path_mode(int type_in, int K_in, int type_out, int K_out, int T, int k, int 
     return (E == 1 ? std::ceil(avg_m / 256.0) * nt < 256.0 : avg_m <= most64) ? kSkinny : kGemm;
   if (q8) {  // (dense)
     const bool long_down = K_out / ((K_in + 255) / 256) > 1024;
-    return (long_down ? T <= 1600 : nt < 16 ? T <= 256 : (T + 63) / 64 * nt <= (!packed ? 310 : K_in <= 2048 ? 560 : 400)) ? kSkinny : kGemm;
+    const int64_t blocks = ((int64_t)T + 63) / 64 * nt, most = !packed ? 310 : K_in <= 2048 ? 560 : 400;
+    return (long_down ? T <= 1600 : nt < 16 ? T <= 256 : blocks <= most) ? kSkinny : kGemm;
   }
   if (avg_m <= (E > 1 ? 96.0 : half ? 800.0 : 1024.0)) return kSkinny;
   if (type_in == EMBER_TYPE_BF16 && type_out == EMBER_TYPE_BF16 && !packed) return kSkinny;
@@ -297,7 +298,8 @@ Layout layout_of(const ember_moe_layer* w, int T, bool tight) {
                      f32_stacks(w->gate_type, w->down_type) ? f32_sh : w->d_ff_shared > 0);
   const bool pack_bf16 = w->prefill_pack && bf16_stacks(w);  // row exponents, also the shared expert's if BF16
   l.mode_shared = w->d_ff_shared > 0 ? path_mode(w->gate_shared_type, w->d, w->down_shared_type, w->d_ff_shared,
-                                                 T, 1, 1, w->prefill_pack && (q8_shared(w) || (pack_bf16 && bf16_shared(w))),
+                                                 T, 1, 1,
+                                                 w->prefill_pack && (q8_shared(w) || (pack_bf16 && bf16_shared(w))),
                                                  false, true)
                                      : kGemv;
   // a shared expert of the routed experts' types rides in the routed decode launches as one more segment

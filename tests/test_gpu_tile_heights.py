@@ -1,8 +1,9 @@
 """The 256-token tiles' heights and the XCDs' runs of work: with k = E every expert holds all T tokens, so T walks
 one tile, the rest of at most 32 rows past whole tiles (left as it is and, every expert ending in one, counted as
 light), and equal tiles in 32-row steps. EMBER_GEMM_SHORT=0 keeps the packs, whose rule for 64-row tiles takes
-layers this small, on 256-row tiles. A row's sums do not depend on its tile, so every row's bits are those of the same token in a call of at most 256 tokens (one tile per expert), and the output holds
-the oracle's bar (utils.cpp:704-748), with the down projection split over K (Q8_0, Q4_K) or not."""
+layers this small, on 256-row tiles. A row's sums do not depend on its tile, so every row's bits are those of the
+same token in a call of at most 256 tokens (one tile per expert), and the output holds the oracle's bar
+(utils.cpp:704-748), with the down projection split over K (Q8_0, Q4_K) or not."""
 import numpy as np
 import pytest
 
@@ -13,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("T", [256, 257, 288, 289, 300, 513, 545, 700])
-@pytest.mark.parametrize("wtype,pack,E", [(em.Q8_0, True, 2), (em.Q8_0, False, 3), (em.Q4_K, True, 2), (em.BF16, True, 2), (em.F16, False, 2)])
+@pytest.mark.parametrize("wtype,pack,E", [(em.Q8_0, True, 2), (em.Q8_0, False, 3), (em.Q4_K, True, 2), (em.BF16, True, 2),
+                                          (em.F16, False, 2)])
 def test_tile_heights(gpu, monkeypatch, wtype, pack, E, T):
     spec = em.LayerSpec(d=256, d_ff=512, E=E, k=E, wtype=wtype, seed=5)
     hl = em.make_host_layer(spec)
